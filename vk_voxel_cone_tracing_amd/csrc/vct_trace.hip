@@ -231,37 +231,44 @@ __device__ __forceinline__ float cone_level(const TraceParams& P, const float po
     return fminf(fmaxf(fmaxf(start_level, cur), min_level), max_level);
 }
 
-// sampleClipmapLinear (voxelConeTracing.frag:329-339). When no lane of the
-// wave has a nonzero texel in its footprints, every lane's sample is exactly
-// zero (a sum of zero texels), which the march accumulates as no change at
-// all (opacity 1 - (1 - 0)^c = 0, colour + 0), so the fetches and the
-// filtering are skipped and zero is returned.
+// sampleClipmapLinear (voxelConeTracing.frag:329-339). A level whose
+// footprints hold no nonzero texel for any lane of the wave contributes
+// exactly zero to every lane (a sum of zero texels), so its fetches and
+// filtering are skipped: the finer level is often empty where the coarser
+// one, whose footprint is eight times as large, is not (1080p frame, 6 x 128^3:
+// diffuse kernel 1513 -> 1260 us, specular 1926 -> 1614 us against one test
+// for both levels). Returns whether any level was fetched; without one `s` is
+// zero for every lane.
 template <bool kHalf>
-__device__ __forceinline__ f4 cone_sample(const typename Vol<kHalf>::T* __restrict__ vol, const TraceParams& P,
-                                          const float pos[3], float cur, const int face[3], const float w[3])
+__device__ __forceinline__ bool cone_sample(const typename Vol<kHalf>::T* __restrict__ vol, const TraceParams& P,
+                                            const float pos[3], float cur, const int face[3], const float w[3], f4& s)
 {
     const int lower = (int)floorf(cur);
     const int upper = (int)ceilf(cur);
     const float fl = cur - floorf(cur);
     float fr_lo[3], fr_hi[3];
     const uint32_t o_lo = footprint(P, pos, lower, fr_lo);
-    bool occ = occupied(P, lower, o_lo);
+    const bool occ_lo = occupied(P, lower, o_lo);
+    bool occ_hi = false;
     uint32_t o_hi = 0;
     if (upper != lower) {
         o_hi = footprint(P, pos, upper, fr_hi);
-        occ = occ || occupied(P, upper, o_hi);
+        occ_hi = occupied(P, upper, o_hi);
     }
-    f4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (!__any(occ)) return s;
-    s = sample_level<kHalf>(vol, P, lower, o_lo, fr_lo, face, w);
-    if (upper != lower) {
-        const f4 hi = sample_level<kHalf>(vol, P, upper, o_hi, fr_hi, face, w);
-        s.x = s.x * (1.0f - fl) + hi.x * fl;
-        s.y = s.y * (1.0f - fl) + hi.y * fl;
-        s.z = s.z * (1.0f - fl) + hi.z * fl;
-        s.w = s.w * (1.0f - fl) + hi.w * fl;
+    const bool any_lo = __any(occ_lo), any_hi = __any(occ_hi);
+    s = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (any_lo) s = sample_level<kHalf>(vol, P, lower, o_lo, fr_lo, face, w);
+    if (any_lo || any_hi) {
+        if (upper != lower) {
+            f4 hi = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (any_hi) hi = sample_level<kHalf>(vol, P, upper, o_hi, fr_hi, face, w);
+            s.x = s.x * (1.0f - fl) + hi.x * fl;
+            s.y = s.y * (1.0f - fl) + hi.y * fl;
+            s.z = s.z * (1.0f - fl) + hi.z * fl;
+            s.w = s.w * (1.0f - fl) + hi.w * fl;
+        }
     }
-    return s;
+    return any_lo || any_hi;
 }
 
 // Front-to-back accumulation of one sample (voxelConeTracing.frag:370-386).
@@ -321,15 +328,17 @@ __device__ f4 trace_cone(const typename Vol<kHalf>::T* __restrict__ vol, const T
 #pragma unroll
         for (int k = 0; k < 3; ++k) pos_b[k] = start[k] + dir[k] * step_b;
         const float cur_b = cone_level(P, pos_b, diam_b, start_level, max_level);
-        const f4 sa = cone_sample<kHalf>(vol, P, pos_a, cur_a, face, w);
-        const f4 sb = cone_sample<kHalf>(vol, P, pos_b, cur_b, face, w);
-        cone_accumulate(P, result, occlusion, sa, cur_a, step, seg);
+        f4 sa, sb;
+        const bool got_a = cone_sample<kHalf>(vol, P, pos_a, cur_a, face, w, sa);
+        const bool got_b = cone_sample<kHalf>(vol, P, pos_b, cur_b, face, w, sb);
+        // a zero sample changes nothing (opacity 1 - 1^c = 0, colour + 0)
+        if (got_a) cone_accumulate(P, result, occlusion, sa, cur_a, step, seg);
         ++steps;
         step = step_b;
         seg = seg_b;
         diameter = diam_b;
         if (!(step < max_dist && occlusion < 1.0f)) break;
-        cone_accumulate(P, result, occlusion, sb, cur_b, step, seg);
+        if (got_b) cone_accumulate(P, result, occlusion, sb, cur_b, step, seg);
         ++steps;
         const float prev = step;
         step += fmaxf(diameter, P.voxel_size) * step_factor;
