@@ -632,31 +632,28 @@ __device__ __forceinline__ void add_block_samples(unsigned long long* samples, u
     }
 }
 
-// Diffuse cones, direct term and mode composition. A workgroup is one 8x8
-// pixel tile; its kWaves waves hold the same pixels and take every kWaves-th
-// cone, leaving the cone results in LDS (one float4 per cone and pixel,
-// dynamic: 16 or 32 KB), where the first wave adds them in cone order, as one
-// lane looping over all cones would. The last wave computes the direct term
-// meanwhile. One lane looping over all cones left the chip partly idle below
-// about a million pixels, and at its end above that (640x360: 229 -> 192 us;
-// 160x90: 118 -> 33 us with sixteen waves). The specular cone, in the modes
-// that trace it, is left to k_trace_specular, which then writes out_s
-// (kSpecPass).
+// Diffuse cones, direct term and mode composition of 8x8 pixel tiles, kWaves
+// waves to a tile. With one wave (four tiles to a workgroup) a lane marches
+// every cone of its pixel. With more, the tile's waves hold the same pixels
+// and take every kWaves-th cone, leaving the cone results in LDS (one float4
+// per cone and pixel, dynamic: 16 or 32 KB), where the first wave adds them in
+// cone order, as the one lane would; the last wave computes the direct term
+// meanwhile. The specular cone, in the modes that trace it, is left to
+// k_trace_specular, which then writes out_s (kSpecPass).
 template <bool kHalf, bool kSpecPass, int kWaves>
-__global__ __launch_bounds__(64 * kWaves) void k_trace(const typename Vol<kHalf>::T* __restrict__ vol, TraceParams P,
-                                               const uint32_t* __restrict__ g_diffuse,
-                                               const uint16_t* __restrict__ g_normal,
-                                               const uint32_t* __restrict__ g_specular,
-                                               const uint16_t* __restrict__ g_emission,
-                                               const float* __restrict__ g_depth, unsigned first_block,
-                                               float4* __restrict__ out_d, float4* __restrict__ out_s,
-                                               unsigned long long* __restrict__ samples)
+__global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void k_trace(
+    const typename Vol<kHalf>::T* __restrict__ vol, TraceParams P, const uint32_t* __restrict__ g_diffuse,
+    const uint16_t* __restrict__ g_normal, const uint32_t* __restrict__ g_specular,
+    const uint16_t* __restrict__ g_emission, const float* __restrict__ g_depth, unsigned first_block,
+    float4* __restrict__ out_d, float4* __restrict__ out_s, unsigned long long* __restrict__ samples)
 {
     extern __shared__ f4 cones[];  // [cone][lane]
     __shared__ f4 direct_term[64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned tiles_x = ((unsigned)P.width + 15u) / 16u;
-    const unsigned block = first_block + xcd_remap(blockIdx.x, gridDim.x), tile = block >> 2, sub = block & 3u;
+    const unsigned block = first_block + xcd_remap(blockIdx.x, gridDim.x);
+    // 16x16-pixel tiles in row order, their 8x8 quarters within
+    const unsigned tile = kWaves == 1 ? block : block >> 2, sub = kWaves == 1 ? (unsigned)wave : block & 3u;
     const int px = (int)(tile % tiles_x) * 16 + (int)(sub & 1u) * 8 + (lane & 7);
     const int py = (int)(tile / tiles_x) * 16 + (int)(sub >> 1) * 8 + (lane >> 3);
     const bool in_image = px < P.width && py < P.height;
@@ -665,45 +662,56 @@ __global__ __launch_bounds__(64 * kWaves) void k_trace(const typename Vol<kHalf>
     const bool surface = depth != 1.0f;
     const int ncones = P.cones32 ? 32 : 16;
     const bool want_diffuse = (P.mode == 4u || P.mode == 5u || P.mode == 7u || P.mode == 8u);
+    const bool want_direct = (P.mode == 4u || P.mode == 5u || P.mode == 8u);
     uint32_t steps = 0;
     PixelIn I;
+    f4 ind = {0.0f, 0.0f, 0.0f, 1.0f};
+    f4 dt = {0.0f, 0.0f, 0.0f, 0.0f};
     if (surface) {
         pixel_in(P, idx, px, py, depth, g_diffuse, g_normal, g_specular, g_emission, I);
         const float aperture = P.cones32 ? 0.628319f : 0.872665f;
-        for (int i = wave; want_diffuse && i < ncones; i += kWaves) {
+        for (int i = kWaves == 1 ? 0 : wave; want_diffuse && i < ncones; i += kWaves) {
             const float* d = P.cones32 ? c_dirs32[i] : c_dirs16[i];
             const float ct = I.normal[0] * d[0] + I.normal[1] * d[1] + I.normal[2] * d[2];
             if (ct < 0.0f) continue;
-            cones[i * 64 + lane] = trace_cone<kHalf>(vol, P, I.start, d, aperture, 30.0f, I.min_level, P.step_factor, steps);
-        }
-        const bool want_direct = (P.mode == 4u || P.mode == 5u || P.mode == 8u);
-        if (wave == kWaves - 1 && want_direct) {
-            float direct[3];
-            if (I.has_emission) {
-                for (int k = 0; k < 3; ++k) direct[k] = I.ef[k];
-            } else {
-                float b[3];
-                brdf(I.normal, I.view, P.light_dir, I.dc, I.sc, I.rough, b);
-                const float visv = trace_visibility(P, I.world);
-                for (int k = 0; k < 3; ++k) direct[k] = b[k] * visv;
-            }
-            direct_term[lane] = {direct[0], direct[1], direct[2], 0.0f};
-        }
-    }
-    __syncthreads();
-    if (wave == 0 && in_image) {
-        float4 dO = make_float4(0.0f, 0.0f, 0.0f, 1.0f);
-        if (surface) {
-            f4 ind = {0.0f, 0.0f, 0.0f, 1.0f};
-            for (int i = 0; want_diffuse && i < ncones; ++i) {
-                const float* d = P.cones32 ? c_dirs32[i] : c_dirs16[i];
-                const float ct = I.normal[0] * d[0] + I.normal[1] * d[1] + I.normal[2] * d[2];
-                if (ct < 0.0f) continue;
-                const f4 c = cones[i * 64 + lane];
+            const f4 c = trace_cone<kHalf>(vol, P, I.start, d, aperture, 30.0f, I.min_level, P.step_factor, steps);
+            if (kWaves == 1) {
                 ind.x += c.x * ct;
                 ind.y += c.y * ct;
                 ind.z += c.z * ct;
                 ind.w += c.w * ct;
+            } else {
+                cones[i * 64 + lane] = c;
+            }
+        }
+        if (want_direct && (kWaves == 1 || wave == kWaves - 1)) {
+            if (I.has_emission) {
+                dt = {I.ef[0], I.ef[1], I.ef[2], 0.0f};
+            } else {
+                float b[3];
+                brdf(I.normal, I.view, P.light_dir, I.dc, I.sc, I.rough, b);
+                const float visv = trace_visibility(P, I.world);
+                dt = {b[0] * visv, b[1] * visv, b[2] * visv, 0.0f};
+            }
+            if (kWaves > 1) direct_term[lane] = dt;
+        }
+    }
+    if (kWaves > 1) __syncthreads();
+    if ((kWaves == 1 || wave == 0) && in_image) {
+        float4 dO = make_float4(0.0f, 0.0f, 0.0f, 1.0f);
+        if (surface) {
+            if (kWaves > 1) {
+                for (int i = 0; want_diffuse && i < ncones; ++i) {
+                    const float* d = P.cones32 ? c_dirs32[i] : c_dirs16[i];
+                    const float ct = I.normal[0] * d[0] + I.normal[1] * d[1] + I.normal[2] * d[2];
+                    if (ct < 0.0f) continue;
+                    const f4 c = cones[i * 64 + lane];
+                    ind.x += c.x * ct;
+                    ind.y += c.y * ct;
+                    ind.z += c.z * ct;
+                    ind.w += c.w * ct;
+                }
+                if (want_direct) dt = direct_term[lane];
             }
             const float inv_n = 1.0f / (float)ncones;
             ind.x *= inv_n;
@@ -714,7 +722,6 @@ __global__ __launch_bounds__(64 * kWaves) void k_trace(const typename Vol<kHalf>
             ind.x *= I.dc[0] * P.diffuse_intensity;
             ind.y *= I.dc[1] * P.diffuse_intensity;
             ind.z *= I.dc[2] * P.diffuse_intensity;
-            const f4 dt = direct_term[lane];
             const float direct[3] = {dt.x, dt.y, dt.z};
             switch (P.mode) {
             case 0: dO = make_float4(I.dc[0], I.dc[1], I.dc[2], 1.0f); break;
@@ -744,7 +751,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_trace(const typename Vol<kHalf>
         out_d[idx] = dO;
         if (!kSpecPass) out_s[idx] = make_float4(0.0f, 0.0f, 0.0f, 1.0f);
     }
-    add_block_samples<kWaves>(samples, steps);
+    add_block_samples<kWaves == 1 ? 4 : kWaves>(samples, steps);
 }
 
 // Specular work ordering. The specular cone's step count is set by the
@@ -1314,10 +1321,14 @@ static size_t spec_tiles(const vct_gbuffer* g)
 // 346 / 159 / 187, 640x360 465 / 342 / 594, 960x540 680 / 675, 1280x720 1094 /
 // 1135 (the 16-lane figures with sixteen waves per tile as well).
 constexpr uint64_t kGroup16Pixels = 1u << 14, kGroup4Pixels = 1u << 19;
-// 8x8 tiles up to which a tile's diffuse cones are spread over sixteen waves:
-// one workgroup of 1024 threads for each of the 256 CUs. 160x90 (240 tiles):
-// 45 us with four waves, 33 with sixteen; 320x180: 73 and 100.
-constexpr unsigned kWideTiles = 256;
+// 8x8 tiles up to which a tile's diffuse cones are spread over sixteen and
+// four waves: sixteen while each of the 256 CUs gets at most one such
+// workgroup (160x90, 240 tiles: 45 us with four waves, 33 with sixteen;
+// 320x180: 73 and 100), four while one wave per tile would be fewer than two
+// rounds of four waves per SIMD (whole RGBA16F ambient-occlusion frame with
+// one / four waves: 320x180 450 / 399 us, 640x360 498 / 482, 960x540 615 / 615,
+// 1280x720 771 / 802, 1920x1080 1212 / 1334: the set-up is repeated per wave).
+constexpr unsigned kWideTiles = 256, kSplitTiles = 8192;
 
 // Workgroups of one k_trace launch: 2^20 (an 8192x8192 image), well below the
 // 2^32 threads a launch may hold.
@@ -1327,11 +1338,11 @@ template <bool kHalf, bool kSpecPass, int kWaves>
 static void launch_diffuse(hipStream_t s, const typename Vol<kHalf>::T* vol, const TraceParams& P,
                            const vct_gbuffer* g, float4* out_d, float4* out_s, unsigned long long* samples)
 {
-    const unsigned blocks = 4u * ((g->width + 15) / 16) * ((g->height + 15) / 16);
-    const size_t lds = (P.cones32 ? 32u : 16u) * 64u * sizeof(f4);
+    const unsigned tiles = ((g->width + 15) / 16) * ((g->height + 15) / 16), blocks = kWaves == 1 ? tiles : 4u * tiles;
+    const size_t lds = kWaves == 1 ? 0 : (P.cones32 ? 32u : 16u) * 64u * sizeof(f4);
     for (unsigned first = 0; first < blocks; first += kTraceBlocks)
         hipLaunchKernelGGL((k_trace<kHalf, kSpecPass, kWaves>), dim3(std::min(kTraceBlocks, blocks - first)),
-                           dim3(64 * kWaves), lds, s, vol, P, g->diffuse, g->normal, g->specular, g->emission, g->depth,
+                           dim3(kWaves == 1 ? 256 : 64 * kWaves), lds, s, vol, P, g->diffuse, g->normal, g->specular, g->emission, g->depth,
                            first, out_d, out_s, samples);
 }
 
@@ -1339,10 +1350,10 @@ template <bool kHalf, bool kSpecPass>
 static void launch_diffuse(hipStream_t s, const typename Vol<kHalf>::T* vol, const TraceParams& P,
                            const vct_gbuffer* g, float4* out_d, float4* out_s, unsigned long long* samples)
 {
-    if (4u * ((g->width + 15) / 16) * ((g->height + 15) / 16) <= kWideTiles)
-        launch_diffuse<kHalf, kSpecPass, 16>(s, vol, P, g, out_d, out_s, samples);
-    else
-        launch_diffuse<kHalf, kSpecPass, 4>(s, vol, P, g, out_d, out_s, samples);
+    const unsigned tiles = 4u * ((g->width + 15) / 16) * ((g->height + 15) / 16);
+    if (tiles <= kWideTiles) launch_diffuse<kHalf, kSpecPass, 16>(s, vol, P, g, out_d, out_s, samples);
+    else if (tiles <= kSplitTiles) launch_diffuse<kHalf, kSpecPass, 4>(s, vol, P, g, out_d, out_s, samples);
+    else launch_diffuse<kHalf, kSpecPass, 1>(s, vol, P, g, out_d, out_s, samples);
 }
 
 template <bool kHalf, int kLanes>
