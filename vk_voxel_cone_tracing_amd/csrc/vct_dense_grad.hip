@@ -77,7 +77,14 @@ __device__ __forceinline__ Corner corner_of(const Pyramid& P, int m, const float
 // sample gradients per channel, which bounds every window sum (see
 // fixed_scale); the per-workgroup accumulators of the coarse levels, shared
 // by many cones, stay in double.
-constexpr int kPoolUnits = 1024;  // a wave's LDS pool for its two live level windows, in 16 B units (16 KB)
+// The splat's workgroup: twelve waves, one workgroup per CU (158 of its 160 KB
+// of LDS). The kernel waits on LDS and memory most of the time, so waves count
+// more than the registers and window space that a third wave per SIMD costs:
+// 8 views of 512x512 at 256^3, forward + backward, 13.9 ms with two workgroups
+// of four waves and 16 KB pools (two waves per SIMD, 234 VGPRs), 13.3 with ten
+// waves and 14 KB, 13.1 with twelve and 12 KB.
+constexpr int kSplatWaves = 12;
+constexpr int kPoolUnits = 768;   // a wave's LDS pool for its two live level windows, in 16 B units (12 KB)
 constexpr int kMaxCopies = 4;     // lane-striped copies of a small window
 constexpr int kCoarseN = 4;       // levels with at most 4^3 interior cells stay in LDS per tile
 constexpr int kCoarseFloats = 24 * (64 + 8 + 1);
@@ -294,6 +301,7 @@ __device__ __forceinline__ void add_channel(float* __restrict__ grad, double* __
         unsafeAtomicAdd(grad + 4ull * idx + ch, (w[0] + w[1] + w[2]) * v);
         return;
     }
+#pragma unroll
     for (int a = 0; a < 3; ++a)
         unsafeAtomicAdd(grad + 4ull * (idx + (unsigned long long)face[a] * P.block[m]) + ch, w[a] * v);
 }
@@ -833,7 +841,7 @@ struct BwdViews {
 // sweep's arithmetic interleaves with other waves' splats, no header, start
 // point or record leaves the kernel, and one launch serves all the views.
 template <bool kFused>
-__global__ __launch_bounds__(256, 2) void k_dense_bwd_splat(Pyramid P, March M, const SweepHeader* __restrict__ hdr,
+__global__ __launch_bounds__(64 * kSplatWaves) void k_dense_bwd_splat(Pyramid P, March M, const SweepHeader* __restrict__ hdr,
                                                          const uint32_t* __restrict__ ctr,
                                                          float4* __restrict__ rec,
                                                          const float4* __restrict__ starts, int width, int height,
@@ -841,19 +849,25 @@ __global__ __launch_bounds__(256, 2) void k_dense_bwd_splat(Pyramid P, March M, 
                                                          const BwdViews VW, uint32_t cap,
                                                          uint32_t* __restrict__ status)
 {
-    __shared__ double s_win[4][2 * kPoolUnits];
+    __shared__ double s_win[kSplatWaves][2 * kPoolUnits];
     __shared__ double s_coarse[kCoarseFloats];
     __shared__ float s_step[kAdjMaxSteps], s_seg[kAdjMaxSteps], s_lvl[kAdjMaxSteps];
     __shared__ float s_corr[kAdjMaxSteps], s_iq[kAdjMaxSteps];
-    __shared__ int s_nsteps;
+    __shared__ int s_nsteps, s_first[kMaxLevels];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const Coarse C = coarse_layout(P);
     int* win = (int*)s_win[wave];
     for (int i = lane; i < 4 * kPoolUnits; i += 64) win[i] = 0;
-    for (int i = tid; i < kCoarseFloats; i += 256) s_coarse[i] = 0.0;
+    for (int i = tid; i < kCoarseFloats; i += 64 * kSplatWaves) s_coarse[i] = 0.0;
     if (tid == 0) {
         const int cnt = step_table(P, M, s_step, s_seg, s_lvl);
         s_nsteps = cnt;
+        // the first step that uses each level (the level rises with the step);
+        // looking for it at every step, in LDS, took 0.3 ms of the 13.1
+        for (int k = cnt - 1; k >= 0; --k) {
+            s_first[(int)floorf(s_lvl[k])] = k;
+            s_first[(int)ceilf(s_lvl[k])] = k;
+        }
         if (kFused && cnt > 0) step_coefs(P, M, cnt, s_step, s_seg, s_lvl, s_corr, s_iq);
     }
     __syncthreads();
@@ -942,11 +956,9 @@ __global__ __launch_bounds__(256, 2) void k_dense_bwd_splat(Pyramid P, March M, 
             for (int j = 0; j < 2; ++j) {
                 if (j >= nlev) break;
                 const int m = j ? hi : lo;
-                // steps k1..k that use level m (the level rises with k)
-                int k1 = k;
-                while (k1 > 0 && (int)ceilf(s_lvl[k1 - 1]) >= m) --k1;
+                if ((m & 1 ? m1 : m0) == m) continue;
+                const int k1 = s_first[m];  // steps k1..k use level m
                 if (m & 1) {
-                    if (m1 == m) continue;
                     if (m1 >= 0 && w1.lds) {
                         wave_lds_sync();
                         flush_window(grad, win, s_coarse, C, P, m1, w1, face, w, lane);
@@ -962,7 +974,6 @@ __global__ __launch_bounds__(256, 2) void k_dense_bwd_splat(Pyramid P, March M, 
                     for (int c = 0; c < 4; ++c) w1.q[c] = fixed_scale(H.gmax[c], k - k1 + 1);
                     m1 = m;
                 } else {
-                    if (m0 == m) continue;
                     if (m0 >= 0 && w0.lds) {
                         wave_lds_sync();
                         flush_window(grad, win, s_coarse, C, P, m0, w0, face, w, lane);
@@ -997,7 +1008,7 @@ __global__ __launch_bounds__(256, 2) void k_dense_bwd_splat(Pyramid P, March M, 
     for (int m = C.first; m < P.nlevels; ++m) {
         const int n = P.n[m], n3 = n * n * n;
         const unsigned long long D = (unsigned long long)n + 2;
-        for (int e = tid; e < 24 * n3; e += 256) {
+        for (int e = tid; e < 24 * n3; e += 64 * kSplatWaves) {
             const float v = (float)s_coarse[coarse_base(C, m) + e];
             if (v == 0.0f) continue;
             const int t = e % n3, ch = (e / n3) & 3, f = e / (4 * n3);
@@ -1130,11 +1141,11 @@ vct_status vct_dense_trace_backward(vct_dense* g, vct_stream stream, const vct_g
     hipStream_t s = (hipStream_t)stream;
     auto* ctr = (uint32_t*)g->bwd_ctr.ptr;
     const uint32_t rec_cap = (uint32_t)(per_tile * chunk / sizeof(float4));
-    // the splat's resident grid: two workgroups per CU (its LDS allows two)
+    // the splat's resident grid: one workgroup per CU (see kSplatWaves)
     int dev = 0, cus = 0;
     VCT_HIP(hipGetDevice(&dev));
     VCT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const uint32_t splat_grid = (uint32_t)std::max(1, 2 * cus);
+    const uint32_t splat_grid = (uint32_t)std::max(1, cus);
     // the sweep takes two cones per workgroup (measured on 16 views of 512 x 512:
     // 48.2 ms forward + backward against 51.4 with all 16 cones per workgroup)
     const uint32_t cone_groups = (uint32_t)((M.ncones + 1) / 2);
@@ -1151,7 +1162,7 @@ vct_status vct_dense_trace_backward(vct_dense* g, vct_stream stream, const vct_g
                                g->data.ptr, P, M, gb->diffuse, gb->normal, gb->depth, (int)gb->width, (int)gb->height,
                                (const float4*)grad_out, t0, rec_cap, (float4*)g->bwd_start.ptr, (float4*)g->bwd_rec.ptr,
                                (dense::SweepHeader*)g->bwd_hdr.ptr, ctr, status, nullptr, 0u);
-        hipLaunchKernelGGL(dense::k_dense_bwd_splat<false>, dim3(splat_grid), dim3(256), 0, s, P, M,
+        hipLaunchKernelGGL(dense::k_dense_bwd_splat<false>, dim3(splat_grid), dim3(64 * dense::kSplatWaves), 0, s, P, M,
                            (const dense::SweepHeader*)g->bwd_hdr.ptr, (const uint32_t*)ctr, (float4*)g->bwd_rec.ptr,
                            (const float4*)g->bwd_start.ptr, (int)gb->width, (int)gb->height, grad_pyramid, ctr + 2,
                            dense::BwdViews{}, 0u, nullptr);
@@ -1195,7 +1206,7 @@ vct_status vct_dense_trace_backward_tapes(vct_dense* g, vct_stream stream, uint3
     int dev = 0, cus = 0;
     VCT_HIP(hipGetDevice(&dev));
     VCT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const uint32_t splat_grid = (uint32_t)std::max(1, 2 * cus);
+    const uint32_t splat_grid = (uint32_t)std::max(1, cus);
     if (T.cap <= (uint32_t)dense::kTapeRegs) {
         // one kernel per kBwdViews views: each slot's reverse sweep, then its splat
         for (uint32_t v0 = 0; v0 < views; v0 += dense::kBwdViews) {
@@ -1215,7 +1226,7 @@ vct_status vct_dense_trace_backward_tapes(vct_dense* g, vct_stream stream, uint3
             }
             auto* ctr = (uint32_t*)((uint8_t*)tapes[v0] + T.ctr_off);
             hipLaunchKernelGGL(dense::k_bwd_reset, dim3(1), dim3(64), 0, s, ctr);
-            hipLaunchKernelGGL(dense::k_dense_bwd_splat<true>, dim3(splat_grid), dim3(256), 0, s, P, M, nullptr, nullptr,
+            hipLaunchKernelGGL(dense::k_dense_bwd_splat<true>, dim3(splat_grid), dim3(64 * dense::kSplatWaves), 0, s, P, M, nullptr, nullptr,
                                nullptr, nullptr, (int)W, (int)H, grad_pyramid, ctr + 2, VW, T.cap, status);
         }
         VCT_HIP(hipGetLastError());
@@ -1237,7 +1248,7 @@ vct_status vct_dense_trace_backward_tapes(vct_dense* g, vct_stream stream, uint3
                            g->data.ptr, P, Mv, gbs[v].diffuse, gbs[v].normal, gbs[v].depth, (int)W, (int)H,
                            (const float4*)grad_outs[v], 0u, 0u, starts, (float4*)base, hdr, ctr, status,
                            (const uint8_t*)base + T.sample_bytes, T.cap);
-        hipLaunchKernelGGL(dense::k_dense_bwd_splat<false>, dim3(splat_grid), dim3(256), 0, s, P, Mv,
+        hipLaunchKernelGGL(dense::k_dense_bwd_splat<false>, dim3(splat_grid), dim3(64 * dense::kSplatWaves), 0, s, P, Mv,
                            (const dense::SweepHeader*)hdr, (const uint32_t*)ctr, (float4*)base, (const float4*)starts,
                            (int)W, (int)H, grad_pyramid, ctr + 2, dense::BwdViews{}, 0u, nullptr);
     }
