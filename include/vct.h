@@ -554,6 +554,14 @@ vct_status vct_dense_tape_bytes(vct_dense* grid, const vct_gbuffer* gbuffer, con
 vct_status vct_dense_trace_tape(vct_dense* grid, vct_stream stream, const vct_gbuffer* gbuffer,
                                 const vct_camera_ubo* camera, const vct_dense_trace_desc* desc, float* out,
                                 unsigned long long* samples_out, void* tape, size_t tape_bytes);
+/* vct_dense_trace (tapes == NULL) or vct_dense_trace_tape over `views` views of
+ * one image size in one call (host arrays of views G-buffers and cameras, and
+ * of device pointers to each view's output and tape, each tape of at least
+ * tape_bytes): the same images and tapes, the views sharing the launches (one
+ * per 16 views). */
+vct_status vct_dense_trace_views(vct_dense* grid, vct_stream stream, uint32_t views, const vct_gbuffer* gbuffers,
+                                 const vct_camera_ubo* cameras, const vct_dense_trace_desc* desc, float* const* outs,
+                                 void* const* tapes, size_t tape_bytes);
 vct_status vct_dense_trace_backward_tape(vct_dense* grid, vct_stream stream, const vct_gbuffer* gbuffer,
                                          const vct_camera_ubo* camera, const vct_dense_trace_desc* desc,
                                          const float* grad_out, void* tape, size_t tape_bytes, float* grad_pyramid,

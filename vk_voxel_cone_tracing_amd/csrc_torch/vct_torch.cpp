@@ -252,17 +252,20 @@ public:
                     tape = torch::empty({per_view * V}, albedo.options().dtype(torch::kUInt8));
             }
         }
+        // all views in one call: they share the launches
+        std::vector<vct_gbuffer> gbs;
+        std::vector<vct_camera_ubo> cams;
+        std::vector<float*> outs;
+        std::vector<void*> tapes;
         for (int64_t v = 0; v < V; ++v) {
-            const vct_gbuffer gb = gbuffer(diffuse, normal, depth, v);
-            const vct_camera_ubo cam = camera(cameras, v);
-            float* o = out.data_ptr<float>() + v * H * W * 4;
-            if (tape.defined())
-                check(vct_dense_trace_tape(slot.grid, s, &gb, &cam, &td, o, nullptr,
-                                           tape.data_ptr<uint8_t>() + v * per_view, (size_t)per_view),
-                      "vct_dense_trace_tape");
-            else
-                check(vct_dense_trace(slot.grid, s, &gb, &cam, &td, o, nullptr), "vct_dense_trace");
+            gbs.push_back(gbuffer(diffuse, normal, depth, v));
+            cams.push_back(camera(cameras, v));
+            outs.push_back(out.data_ptr<float>() + v * H * W * 4);
+            if (tape.defined()) tapes.push_back(tape.data_ptr<uint8_t>() + v * per_view);
         }
+        check(vct_dense_trace_views(slot.grid, s, (uint32_t)V, gbs.data(), cams.data(), &td, outs.data(),
+                                    tape.defined() ? tapes.data() : nullptr, (size_t)per_view),
+              "vct_dense_trace_views");
         if (tape.defined()) {
             ctx->saved_data["tape"] = tape;
             ctx->saved_data["tape_view_bytes"] = per_view;
