@@ -417,7 +417,7 @@ vct_status vct_destroy(vct_ctx* c)
                             &c->offsets, &c->scan_tmp, &c->totals, &c->rec_key[0], &c->rec_key[1], &c->rec_idx[0],
                             &c->rec_idx[1], &c->rec_val, &c->sort_tmp, &c->staging, &c->materials_flat,
                             &c->svo.frags, &c->svo.pool, &c->svo.counters, &c->spec_perm, &c->svo.cells,
-                            &c->svo.grids, &c->svo.bricks, &c->soup_uv};
+                            &c->svo.grids, &c->svo.bricks, &c->soup_uv, &c->svo.top};
     for (DeviceBuffer* b : bufs) release(*b);
     if (c->pinned) (void)hipHostFree(c->pinned);
     if (c->pinned_word) (void)hipHostFree(c->pinned_word);

@@ -82,7 +82,16 @@ struct SvoState {
     DeviceBuffer grids;      // dense node-colour grid of every depth (brick builder)
     DeviceBuffer bricks;     // 27 RGBA8 per node
     bool bricks_built = false;
+    // The octree trace's walk table: for every cell of 2^kSvoTopBits voxels of
+    // the built octree, the walk's state on entering it (child block, colour);
+    // 2^top_bits cells per axis, top_bits 0 without a table (small octrees).
+    DeviceBuffer top;
+    uint32_t top_bits = 0;
 };
+
+// log2 of the walk table's cell edge: the coarsest level an octree sample asks
+// for is 5 (six levels), so every walk passes through its cell.
+constexpr uint32_t kSvoTopBits = 5;
 
 }  // namespace vct
 

@@ -353,6 +353,20 @@ __global__ __launch_bounds__(256) void k_svo_mip(uint2* __restrict__ pool, uint3
     pool[begin + i].y = pack_raw(f4{s[0], s[1], s[2], s[3]});
 }
 
+// The walk of every cell of 2^kSvoTopBits voxels, from the root: the state a
+// sample's walk has on entering the cell, or where it ends above it.
+__global__ __launch_bounds__(256) void k_svo_top(const uint2* __restrict__ pool, uint32_t L, uint32_t bits,
+                                                 uint2* __restrict__ top)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, mask = (1u << bits) - 1u;
+    if (i >= 1u << (3u * bits)) return;
+    uint32_t p[3] = {(i & mask) << kSvoTopBits, ((i >> bits) & mask) << kSvoTopBits, (i >> (2u * bits)) << kSvoTopBits};
+    uint32_t r;
+    const uint32_t idx = walk(pool, p, 1u << L, 1u << kSvoTopBits, r);
+    const uint2 node = pool[idx];
+    top[i] = make_uint2(r == 1u << kSvoTopBits ? node.x & 0x7fffffffu : 0u, node.y);
+}
+
 static LightParams make_light(const vct_shadow_map* shadow, const vct_directional_light_desc* light,
                               const vct_directional_light_shadow_desc* ls)
 {
@@ -694,6 +708,14 @@ vct_status vct_svo_build(vct_ctx* c, vct_stream stream)
         if (depth < 1 || depth > level_begin.size()) continue;
         hipLaunchKernelGGL(k_svo_mip, dim3(blocks_for(level_num[depth - 1])), dim3(256), 0, s, pool,
                            level_begin[depth - 1], level_num[depth - 1]);
+    }
+    // the octree trace's walk table
+    c->svo.top_bits = L > kSvoTopBits ? L - kSvoTopBits : 0u;
+    if (c->svo.top_bits) {
+        const size_t cells = (size_t)1 << (3u * c->svo.top_bits);
+        VCT_TRY(ensure(c->svo.top, sizeof(uint2) * cells));
+        hipLaunchKernelGGL(k_svo_top, dim3(blocks_for(cells)), dim3(256), 0, s, (const uint2*)pool, L, c->svo.top_bits,
+                           (uint2*)c->svo.top.ptr);
     }
     VCT_HIP(hipGetLastError());
     c->svo.depths = (uint32_t)level_begin.size();
