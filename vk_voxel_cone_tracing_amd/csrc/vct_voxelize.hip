@@ -20,6 +20,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "vct_expand.hpp"
 #include "vct_internal.hpp"
 #include "vct_raster.hpp"
 #include "vct_shadow.hpp"
@@ -100,22 +101,28 @@ struct LevelSet {
     uint32_t keep_mask;  // bit l: clip level l keeps its stored alpha (RGBA16F after vct_begin_radiance_level)
 };
 
-// counts[slot * ntris + t]: the work items (cells x samples) of triangle t in
-// the slot's level (grid: triangles x slots).
-__global__ void k_count(const float* __restrict__ pos, uint32_t ntris, LevelSet S,
-                        unsigned long long* __restrict__ counts)
+// The work items (cells x samples) of triangle t in the slot's level (grid:
+// triangles x slots): their prefix within the block of 256 triangles, and the
+// block's sum. With k_total this is the whole scan, 10 us in two launches (a
+// library scan of the counts: 18 us in four).
+__global__ __launch_bounds__(kExpandBlock) void k_count(const float* __restrict__ pos, uint32_t ntris, LevelSet S,
+                                                        uint32_t* __restrict__ in_block,
+                                                        unsigned long long* __restrict__ block_sums)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int slot = (int)blockIdx.y;
-    if (t >= ntris) return;
-    const VoxParams& P = S.P[slot];
-    float p[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) p[k] = pos[9u * t + k];
-    TriSetup s;
+    const uint32_t t = blockIdx.x * kExpandBlock + threadIdx.x, slot = blockIdx.y;
     unsigned long long n = 0;
-    if (tri_setup(p, P.voxel_size, P.lo, P.hi, s)) n = (unsigned long long)s.nu * s.nv * (unsigned long long)P.samples;
-    counts[(size_t)slot * ntris + t] = n;
+    if (t < ntris) {
+        const VoxParams& P = S.P[slot];
+        float p[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) p[k] = pos[9u * t + k];
+        TriSetup s;
+        if (tri_setup(p, P.voxel_size, P.lo, P.hi, s))
+            n = (unsigned long long)s.nu * s.nv * (unsigned long long)P.samples;
+    }
+    const uint32_t b = slot * gridDim.x + blockIdx.x;
+    const unsigned long long below = expand_block(n, &block_sums[b]);
+    in_block[(size_t)b * kExpandBlock + threadIdx.x] = (uint32_t)below;
 }
 
 // The work items of the slots are numbered consecutively, each slot starting
@@ -134,15 +141,17 @@ constexpr int kTotRec = 32, kTotWords = kTotRec + 1;
 static_assert(kTotC + kMaxLevels <= kTotRec, "slot table overlaps the record counter");
 static_assert(8u * kTotWords <= kPinnedWordBytes, "totals read back into the pinned landing slot");
 
-__global__ void k_total(const unsigned long long* __restrict__ counts, const unsigned long long* __restrict__ offsets,
-                        uint32_t ntris, int nslots, unsigned long long* __restrict__ totals)
+// Scans the block sums (nblocks per slot) and writes the totals.
+__global__ __launch_bounds__(1024) void k_total(unsigned long long* __restrict__ blocks, uint32_t nblocks, int nslots,
+                                                unsigned long long* __restrict__ totals)
 {
-    const size_t n = (size_t)ntris * (size_t)nslots;
-    const unsigned long long all = n ? offsets[n - 1] + counts[n - 1] : 0ull;
+    const unsigned long long all = expand_scan(blocks, nblocks * (uint32_t)nslots);
+    __syncthreads();
+    if (threadIdx.x != 0) return;
     unsigned long long a = 0;
     for (int k = 0; k < nslots; ++k) {
-        const unsigned long long u = offsets[(size_t)k * ntris];
-        const unsigned long long next = k + 1 < nslots ? offsets[(size_t)(k + 1) * ntris] : all;
+        const unsigned long long u = nblocks ? blocks[(size_t)k * nblocks] : 0ull;
+        const unsigned long long next = k + 1 < nslots && nblocks ? blocks[(size_t)(k + 1) * nblocks] : all;
         totals[kTotA + k] = a;
         totals[kTotU + k] = u;
         totals[kTotC + k] = next - u;
@@ -165,9 +174,8 @@ __host__ __device__ inline uint32_t work_bits(unsigned long long n)
 
 // The slot of work item wi (wave-uniform, see k_total), its position in the
 // unpadded numbering (the work index the injection's record keys carry) and
-// its triangle (a search within the slot's triangles: with tens of thousands
-// of triangles a full search per lane is cheaper than narrowing it with
-// block-uniform searches first). valid is false for a slot's padding.
+// its triangle. The whole wave calls it with consecutive items from a multiple
+// of 64. valid is false for a slot's padding.
 struct WorkItem {
     int slot;
     bool valid;
@@ -175,26 +183,21 @@ struct WorkItem {
     uint32_t sample;  // index of the (cell, sample) within the triangle
 };
 
-__device__ __forceinline__ WorkItem work_item(const unsigned long long* __restrict__ offsets,
-                                              const unsigned long long* __restrict__ totals, uint32_t ntris, int nslots,
-                                              unsigned long long wi)
+__device__ __forceinline__ WorkItem work_item(const Expansion& E, const unsigned long long* __restrict__ totals,
+                                              uint32_t ntris, int nslots, unsigned long long wi)
 {
     int slot = 0;
     for (int k = 1; k < nslots; ++k) slot += wi >= totals[kTotA + k] ? 1 : 0;
     slot = __builtin_amdgcn_readfirstlane(slot);  // one slot per wave
     WorkItem it;
     it.slot = slot;
-    const unsigned long long local = wi - totals[kTotA + slot];
-    it.valid = local < totals[kTotC + slot];
-    it.t = 0;
-    it.sample = 0;
-    if (it.valid) {
-        const unsigned long long index = totals[kTotU + slot] + local;
-        const uint32_t base = (uint32_t)slot * ntris;
-        const uint32_t j = work_triangle(offsets, base, base + ntris - 1u, index);
-        it.t = j - base;
-        it.sample = (uint32_t)(index - offsets[j]);
-    }
+    const unsigned long long local = wi - totals[kTotA + slot], count = totals[kTotC + slot], u = totals[kTotU + slot];
+    it.valid = local < count;
+    const uint32_t nblocks = (ntris + kExpandBlock - 1u) / kExpandBlock, base = (uint32_t)slot * nblocks;
+    const Expansion slot_items{E.in_block + (size_t)base * kExpandBlock, E.block + base};
+    const unsigned long long local0 = local - (threadIdx.x & 63u);  // a wave's first item is valid
+    it.t = wave_triangle(slot_items, ntris, u + local0, u + count - 1ull);
+    it.sample = it.valid ? (uint32_t)(u + local - slot_items(it.t)) : 0u;
     return it;
 }
 
@@ -206,14 +209,14 @@ __device__ __forceinline__ unsigned long long work_index(const unsigned long lon
 }
 
 __global__ __launch_bounds__(256) void k_raster_opacity(const float* __restrict__ pos,
-                                                        const unsigned long long* __restrict__ offsets, uint32_t ntris,
+                                                        Expansion E, uint32_t ntris,
                                                         const unsigned long long* __restrict__ totals, LevelSet S,
                                                         TexInputs T, uint32_t* __restrict__ vol)
 {
     const unsigned long long n = totals[0];
     const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
     for (unsigned long long wi = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; wi < n; wi += stride) {
-        const WorkItem it = work_item(offsets, totals, ntris, S.n, wi);
+        const WorkItem it = work_item(E, totals, ntris, S.n, wi);
         if (!it.valid) continue;
         const VoxParams P = S.P[it.slot];
         const uint32_t t = it.t;
@@ -244,107 +247,140 @@ struct Record {
 };
 
 __global__ __launch_bounds__(256) void k_raster_inject(const float* __restrict__ pos, const float* __restrict__ nrm,
-                                                       TexInputs T, const unsigned long long* __restrict__ offsets,
-                                                       uint32_t ntris, unsigned long long* __restrict__ totals,
+                                                       TexInputs T, Expansion E, uint32_t ntris,
+                                                       unsigned long long* __restrict__ totals,
                                                        LevelSet S, LightParams L,
                                                        unsigned long long* __restrict__ keys,
                                                        uint32_t* __restrict__ idx, Record* __restrict__ vals,
                                                        uint32_t cap)
 {
 #pragma clang fp contract(off)
+    __shared__ uint32_t wave_records[4];
+    __shared__ unsigned long long block_first;
     const unsigned long long n = totals[0];
     if (n > 0xffffffffull) return;  // record keys hold 32 bits of work index; the host reports it
     const uint32_t wbits = work_bits(n);
     const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
-    for (unsigned long long wi = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; wi < n; wi += stride) {
-        const WorkItem it = work_item(offsets, totals, ntris, S.n, wi);
-        if (!it.valid) continue;
-        const VoxParams P = S.P[it.slot];
-        const float box_lo[3] = {S.box_lo[it.slot][0], S.box_lo[it.slot][1], S.box_lo[it.slot][2]};
-        const float box_hi[3] = {S.box_hi[it.slot][0], S.box_hi[it.slot][1], S.box_hi[it.slot][2]};
-        const uint32_t t = it.t;
-        float p[9];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) p[k] = pos[9u * t + k];
-        TriSetup s;
-        if (!tri_setup(p, P.voxel_size, P.lo, P.hi, s)) continue;
-        float fp[3];
-        double lam[3];
-        if (!tri_sample(p, s, P.voxel_size, P.samples, it.sample, fp, lam)) continue;
-        if (fp[0] < box_lo[0] || fp[1] < box_lo[1] || fp[2] < box_lo[2] || fp[0] > box_hi[0] || fp[1] > box_hi[1] ||
-            fp[2] > box_hi[2])
-            continue;
-        const vct_gltf_material& m = T.mats[T.mat[t]];
-        float uv[2] = {0.0f, 0.0f};
-        if (T.tex) {
-            // msaaInjectRadiance.frag:73-74: occlusion-texture discard
-            interp_uv(T.uv + 6u * t, lam, uv);
-            if (occluded(T, m, uv)) continue;
-        }
-        int ic[3];
-        image_coords(P, fp, ic);
+    // The records' places in the buffer come from one atomic per workgroup and
+    // trip: the counter is one address, which takes some 90 million atomics a
+    // second, and one per wave was the kernel's bound (128^3 x 6 levels, 21 260
+    // triangles: 189 -> 115 us).
+    for (unsigned long long base = (unsigned long long)blockIdx.x * 256u; base < n; base += stride) {
+        const unsigned long long wi = base + threadIdx.x;
         Record out[6];
         int faces[6];
-        int nout = 0;
-        if (m.emissive_factor[0] > 0.0f || m.emissive_factor[1] > 0.0f || m.emissive_factor[2] > 0.0f) {
-            // msaaInjectRadiance.frag:76-86; the emissive texture adds to the factor
-            float em[3] = {m.emissive_factor[0], m.emissive_factor[1], m.emissive_factor[2]};
-            if (has_texture(T, m.emissive_texture)) {
-                const f4 te = sample_texture(T.tex[m.emissive_texture], uv);
-                em[0] = em[0] + te.x;
-                em[1] = em[1] + te.y;
-                em[2] = em[2] + te.z;
+        int ic[3] = {0, 0, 0};
+        int nout = 0, slot = 0;
+        // one item: its records in `out`, `nout` of them
+        auto raster = [&]() {
+            const WorkItem it = work_item(E, totals, ntris, S.n, wi);
+            slot = it.slot;
+            if (!it.valid) return;
+            const VoxParams P = S.P[it.slot];
+            const float box_lo[3] = {S.box_lo[it.slot][0], S.box_lo[it.slot][1], S.box_lo[it.slot][2]};
+            const float box_hi[3] = {S.box_hi[it.slot][0], S.box_hi[it.slot][1], S.box_hi[it.slot][2]};
+            const uint32_t t = it.t;
+            float p[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) p[k] = pos[9u * t + k];
+            TriSetup s;
+            if (!tri_setup(p, P.voxel_size, P.lo, P.hi, s)) return;
+            float fp[3];
+            double lam[3];
+            if (!tri_sample(p, s, P.voxel_size, P.samples, it.sample, fp, lam)) return;
+            if (fp[0] < box_lo[0] || fp[1] < box_lo[1] || fp[2] < box_lo[2] || fp[0] > box_hi[0] || fp[1] > box_hi[1] ||
+                fp[2] > box_hi[2])
+                return;
+            const vct_gltf_material& m = T.mats[T.mat[t]];
+            float uv[2] = {0.0f, 0.0f};
+            if (T.tex) {
+                // msaaInjectRadiance.frag:73-74: occlusion-texture discard
+                interp_uv(T.uv + 6u * t, lam, uv);
+                if (occluded(T, m, uv)) return;
             }
-            Record e = {fminf(fmaxf(em[0], 0.0f), 1.0f), fminf(fmaxf(em[1], 0.0f), 1.0f),
-                        fminf(fmaxf(em[2], 0.0f), 1.0f)};
-            for (int f = 0; f < 6; ++f) {
-                out[f] = e;
-                faces[f] = f;
+            image_coords(P, fp, ic);
+            if (m.emissive_factor[0] > 0.0f || m.emissive_factor[1] > 0.0f || m.emissive_factor[2] > 0.0f) {
+                // msaaInjectRadiance.frag:76-86; the emissive texture adds to the factor
+                float em[3] = {m.emissive_factor[0], m.emissive_factor[1], m.emissive_factor[2]};
+                if (has_texture(T, m.emissive_texture)) {
+                    const f4 te = sample_texture(T.tex[m.emissive_texture], uv);
+                    em[0] = em[0] + te.x;
+                    em[1] = em[1] + te.y;
+                    em[2] = em[2] + te.z;
+                }
+                Record e = {fminf(fmaxf(em[0], 0.0f), 1.0f), fminf(fmaxf(em[1], 0.0f), 1.0f),
+                            fminf(fmaxf(em[2], 0.0f), 1.0f)};
+                for (int f = 0; f < 6; ++f) {
+                    out[f] = e;
+                    faces[f] = f;
+                }
+                nout = 6;
+            } else {
+                // msaaInjectRadiance.frag:131-153
+                const float* n0 = nrm + 9u * t;
+                float ni[3];
+                for (int k = 0; k < 3; ++k)
+                    ni[k] = (float)(lam[0] * (double)n0[k] + lam[1] * (double)n0[3 + k] + lam[2] * (double)n0[6 + k]);
+                const float len = sqrtf(ni[0] * ni[0] + ni[1] * ni[1] + ni[2] * ni[2]);
+                const float nn[3] = {ni[0] / len, ni[1] / len, ni[2] / len};
+                float ndl = nn[0] * L.dir[0] + nn[1] * L.dir[1] + nn[2] * L.dir[2];
+                ndl = fminf(fmaxf(ndl, 0.001f), 1.0f);
+                const float vis = visibility(L, fp, P.quirks);
+                float lc[3];
+                for (int k = 0; k < 3; ++k) lc[k] = ndl * vis * L.color[k] * L.intensity;
+                if (lc[0] == 0.0f && lc[1] == 0.0f && lc[2] == 0.0f) return;
+                // msaaInjectRadiance.frag:131-136: the base-colour texture scales the factor
+                float col[4] = {m.base_color_factor[0], m.base_color_factor[1], m.base_color_factor[2],
+                                m.base_color_factor[3]};
+                if (has_texture(T, m.base_color_texture)) {
+                    const f4 tb = sample_texture(T.tex[m.base_color_texture], uv);
+                    col[0] = col[0] * tb.x;
+                    col[1] = col[1] * tb.y;
+                    col[2] = col[2] * tb.z;
+                    col[3] = col[3] * tb.w;
+                }
+                float rad[3];
+                for (int k = 0; k < 3; ++k) rad[k] = fminf(fmaxf(lc[k] * col[k] * col[3], 0.0f), 1.0f);
+                const int face[3] = {(-nn[0] > 0.0f) ? 0 : 1, (-nn[1] > 0.0f) ? 2 : 3, (-nn[2] > 0.0f) ? 4 : 5};
+                for (int k = 0; k < 3; ++k) {
+                    const float w = fabsf(nn[k]);
+                    out[k] = {rad[0] * w, rad[1] * w, rad[2] * w};
+                    faces[k] = face[k];
+                }
+                nout = 3;
             }
-            nout = 6;
-        } else {
-            // msaaInjectRadiance.frag:131-153
-            const float* n0 = nrm + 9u * t;
-            float ni[3];
-            for (int k = 0; k < 3; ++k)
-                ni[k] = (float)(lam[0] * (double)n0[k] + lam[1] * (double)n0[3 + k] + lam[2] * (double)n0[6 + k]);
-            const float len = sqrtf(ni[0] * ni[0] + ni[1] * ni[1] + ni[2] * ni[2]);
-            const float nn[3] = {ni[0] / len, ni[1] / len, ni[2] / len};
-            float ndl = nn[0] * L.dir[0] + nn[1] * L.dir[1] + nn[2] * L.dir[2];
-            ndl = fminf(fmaxf(ndl, 0.001f), 1.0f);
-            const float vis = visibility(L, fp, P.quirks);
-            float lc[3];
-            for (int k = 0; k < 3; ++k) lc[k] = ndl * vis * L.color[k] * L.intensity;
-            if (lc[0] == 0.0f && lc[1] == 0.0f && lc[2] == 0.0f) continue;
-            // msaaInjectRadiance.frag:131-136: the base-colour texture scales the factor
-            float col[4] = {m.base_color_factor[0], m.base_color_factor[1], m.base_color_factor[2],
-                            m.base_color_factor[3]};
-            if (has_texture(T, m.base_color_texture)) {
-                const f4 tb = sample_texture(T.tex[m.base_color_texture], uv);
-                col[0] = col[0] * tb.x;
-                col[1] = col[1] * tb.y;
-                col[2] = col[2] * tb.z;
-                col[3] = col[3] * tb.w;
-            }
-            float rad[3];
-            for (int k = 0; k < 3; ++k) rad[k] = fminf(fmaxf(lc[k] * col[k] * col[3], 0.0f), 1.0f);
-            const int face[3] = {(-nn[0] > 0.0f) ? 0 : 1, (-nn[1] > 0.0f) ? 2 : 3, (-nn[2] > 0.0f) ? 4 : 5};
-            for (int k = 0; k < 3; ++k) {
-                const float w = fabsf(nn[k]);
-                out[k] = {rad[0] * w, rad[1] * w, rad[2] * w};
-                faces[k] = face[k];
-            }
-            nout = 3;
+        };
+        if (wi < n) raster();  // n is a multiple of 64: whole waves
+        slot = __builtin_amdgcn_readfirstlane(slot);
+        const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+        uint32_t upto = (uint32_t)nout;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t u = __shfl_up(upto, off, 64);
+            if (lane >= (uint32_t)off) upto += u;
         }
-        const unsigned long long first = atomicAdd(&totals[kTotRec], (unsigned long long)nout);
-        const unsigned long long index = work_index(totals, it.slot, wi);
-        for (int j = 0; j < nout; ++j) {
-            const unsigned long long r = first + (unsigned long long)j;
-            if (r >= cap) break;  // capacity is checked on the host from the counter
-            const size_t addr = vol_index(P.D, P.clip_level, faces[j], ic[0], ic[1], ic[2]);
-            keys[r] = ((unsigned long long)addr << wbits) | index;
-            idx[r] = (uint32_t)r;
-            vals[r] = out[j];
+        __syncthreads();  // the previous trip's reads of the shared words are done
+        if (lane == 63u) wave_records[wave] = upto;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint32_t all = wave_records[0] + wave_records[1] + wave_records[2] + wave_records[3];
+            block_first = all ? atomicAdd(&totals[kTotRec], (unsigned long long)all) : 0ull;
+        }
+        __syncthreads();
+        if (nout) {
+            unsigned long long first = block_first + upto - (uint32_t)nout;
+            for (uint32_t w = 0; w < wave; ++w) first += wave_records[w];
+            const unsigned long long index = work_index(totals, slot, wi);
+            const int D = S.P[slot].D, level = S.P[slot].clip_level;
+#pragma unroll
+            for (int j = 0; j < 6; ++j) {
+                const unsigned long long r = first + (unsigned long long)j;
+                if (j >= nout || r >= cap) break;  // capacity is checked on the host from the counter
+                const size_t addr = vol_index(D, level, faces[j], ic[0], ic[1], ic[2]);
+                keys[r] = ((unsigned long long)addr << wbits) | index;
+                idx[r] = (uint32_t)r;
+                vals[r] = out[j];
+            }
         }
     }
 }
@@ -538,29 +574,23 @@ static vct_status make_level_set(vct_ctx* c, const vct_voxelization_desc* descs,
     return VCT_OK;
 }
 
-// Per-(level, triangle) counts, their exclusive scan and the totals.
-static vct_status expand(vct_ctx* c, hipStream_t s, const TriSoup& soup, const LevelSet& S)
+// The expansion of the (level, triangle) pairs and the totals.
+static vct_status expand(vct_ctx* c, hipStream_t s, const TriSoup& soup, const LevelSet& S, Expansion* E)
 {
-    const size_t n = (size_t)soup.count * (size_t)S.n;
-    if (n > 0x7fffffffull) return fail(VCT_ERR_CAPACITY, "%zu triangle-level pairs exceed 2^31", n);
-    VCT_TRY(ensure(c->counts, 8u * (n ? n : 1)));
+    const uint32_t nblocks = (soup.count + kExpandBlock - 1u) / kExpandBlock;
+    const size_t n = (size_t)nblocks * (size_t)S.n;
+    if ((size_t)soup.count * (size_t)S.n > 0x7fffffffull)
+        return fail(VCT_ERR_CAPACITY, "%zu triangle-level pairs exceed 2^31", (size_t)soup.count * (size_t)S.n);
+    VCT_TRY(ensure(c->counts, 4u * (n ? n : 1) * kExpandBlock));
     VCT_TRY(ensure(c->offsets, 8u * (n ? n : 1)));
     VCT_TRY(ensure(c->totals, 8u * kTotWords));
-    if (n) {
-        hipLaunchKernelGGL(k_count, dim3((soup.count + 255) / 256, (unsigned)S.n), dim3(256), 0, s, soup.pos,
-                           soup.count, S, (unsigned long long*)c->counts.ptr);
-        VCT_HIP(hipGetLastError());
-        size_t tmp = 0;
-        VCT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, (unsigned long long*)c->counts.ptr,
-                                                 (unsigned long long*)c->offsets.ptr, (int)n, s));
-        VCT_TRY(ensure(c->scan_tmp, tmp));
-        VCT_HIP(hipcub::DeviceScan::ExclusiveSum(c->scan_tmp.ptr, tmp, (unsigned long long*)c->counts.ptr,
-                                                 (unsigned long long*)c->offsets.ptr, (int)n, s));
-    }
-    hipLaunchKernelGGL(k_total, dim3(1), dim3(1), 0, s, (const unsigned long long*)c->counts.ptr,
-                       (const unsigned long long*)c->offsets.ptr, soup.count, S.n,
+    if (n)
+        hipLaunchKernelGGL(k_count, dim3(nblocks, (unsigned)S.n), dim3(kExpandBlock), 0, s, soup.pos, soup.count, S,
+                           (uint32_t*)c->counts.ptr, (unsigned long long*)c->offsets.ptr);
+    hipLaunchKernelGGL(k_total, dim3(1), dim3(1024), 0, s, (unsigned long long*)c->offsets.ptr, nblocks, S.n,
                        (unsigned long long*)c->totals.ptr);
     VCT_HIP(hipGetLastError());
+    *E = {(const uint32_t*)c->counts.ptr, (const unsigned long long*)c->offsets.ptr};
     return VCT_OK;
 }
 
@@ -573,11 +603,11 @@ static vct_status voxelize_levels(vct_ctx* c, hipStream_t s, const vct_mesh* mes
     TriSoup soup;
     VCT_TRY(run_vertex_stage(c, s, mesh, &soup));
     if (!soup.count) return VCT_OK;
-    VCT_TRY(expand(c, s, soup, S));
+    Expansion E;
+    VCT_TRY(expand(c, s, soup, S, &E));
     // grid-stride over a device-side total: no host synchronisation
     const TexInputs T{soup.uv, soup.mat, mesh->materials, soup.tex, soup.tex_count};
-    hipLaunchKernelGGL(k_raster_opacity, dim3(8192), dim3(256), 0, s, soup.pos,
-                       (const unsigned long long*)c->offsets.ptr, soup.count,
+    hipLaunchKernelGGL(k_raster_opacity, dim3(8192), dim3(256), 0, s, soup.pos, E, soup.count,
                        (const unsigned long long*)c->totals.ptr, S, T, (uint32_t*)c->opacity.ptr);
     VCT_HIP(hipGetLastError());
     return VCT_OK;
@@ -603,7 +633,8 @@ static vct_status inject_levels(vct_ctx* c, hipStream_t s, const vct_mesh* mesh,
     TriSoup soup;
     VCT_TRY(run_vertex_stage(c, s, mesh, &soup));
     if (!soup.count) return VCT_OK;
-    VCT_TRY(expand(c, s, soup, S));
+    Expansion E;
+    VCT_TRY(expand(c, s, soup, S, &E));
 
     LightParams L;
     {
@@ -635,8 +666,8 @@ static vct_status inject_levels(vct_ctx* c, hipStream_t s, const vct_mesh* mesh,
     const TexInputs T{soup.uv, soup.mat, mesh->materials, soup.tex, soup.tex_count};
     for (int attempt = 0;; ++attempt) {
         const uint32_t cap = c->inject_cap;
-        hipLaunchKernelGGL(k_raster_inject, dim3(8192), dim3(256), 0, s, soup.pos, soup.nrm, T,
-                           (const unsigned long long*)c->offsets.ptr, soup.count, (unsigned long long*)c->totals.ptr,
+        hipLaunchKernelGGL(k_raster_inject, dim3(8192), dim3(256), 0, s, soup.pos, soup.nrm, T, E, soup.count,
+                           (unsigned long long*)c->totals.ptr,
                            S, L, (unsigned long long*)c->rec_key[0].ptr, (uint32_t*)c->rec_idx[0].ptr,
                            (Record*)c->rec_val.ptr, cap);
         VCT_HIP(hipGetLastError());
