@@ -98,7 +98,9 @@ vct_status upload_small(vct_ctx* ctx, hipStream_t s, DeviceBuffer& dst, const vo
 }
 
 // ---------------------------------------------------------------------------
-// Vertex stage: one thread per triangle of the flattened draw list.
+// Vertex stage: one thread per triangle of the flattened draw list. Normals
+// and texture coordinates are written where the pass reads them only (null
+// outputs): they are 60 of a triangle's 100 bytes.
 
 struct DevPrim {
     uint32_t first_index;
@@ -131,13 +133,16 @@ __global__ void k_vertex_stage(const float* __restrict__ positions, const float*
     for (int k = 0; k < 3; ++k) {
         uint32_t vi = (uint32_t)((int64_t)indices[pr.first_index + 3u * local + (uint32_t)k] + pr.vertex_offset);
         float px = positions[3u * vi], py = positions[3u * vi + 1], pz = positions[3u * vi + 2];
-        float nx = normals[3u * vi], ny = normals[3u * vi + 1], nz = normals[3u * vi + 2];
-        for (int r = 0; r < 3; ++r) {
+        for (int r = 0; r < 3; ++r)
             out_pos[9u * t + 3 * k + r] = ((m[r] * px + m[4 + r] * py) + m[8 + r] * pz) + m[12 + r];
-            out_nrm[9u * t + 3 * k + r] = (it[r] * nx + it[4 + r] * ny) + it[8 + r] * nz;
+        if (out_nrm) {
+            float nx = normals[3u * vi], ny = normals[3u * vi + 1], nz = normals[3u * vi + 2];
+            for (int r = 0; r < 3; ++r) out_nrm[9u * t + 3 * k + r] = (it[r] * nx + it[4 + r] * ny) + it[8 + r] * nz;
         }
-        out_uv[6u * t + 2 * k] = texcoords ? texcoords[2u * vi] : 0.0f;
-        out_uv[6u * t + 2 * k + 1] = texcoords ? texcoords[2u * vi + 1] : 0.0f;
+        if (out_uv) {
+            out_uv[6u * t + 2 * k] = texcoords ? texcoords[2u * vi] : 0.0f;
+            out_uv[6u * t + 2 * k + 1] = texcoords ? texcoords[2u * vi + 1] : 0.0f;
+        }
     }
     out_mat[t] = pr.material_index;
 }
@@ -209,7 +214,8 @@ static vct_status check_textures(vct_ctx* ctx, hipStream_t s, const vct_mesh* me
     return VCT_OK;
 }
 
-vct_status run_vertex_stage(vct_ctx* ctx, hipStream_t s, const vct_mesh* mesh, TriSoup* out, TextureUse use)
+vct_status run_vertex_stage(vct_ctx* ctx, hipStream_t s, const vct_mesh* mesh, TriSoup* out, TextureUse use,
+                            bool normals)
 {
     if (!mesh || !mesh->positions || !mesh->normals || !mesh->indices || !mesh->node_matrices || !mesh->materials)
         return fail(VCT_ERR_INVALID_ARGUMENT, "mesh buffers must be non-null");
@@ -266,13 +272,13 @@ vct_status run_vertex_stage(vct_ctx* ctx, hipStream_t s, const vct_mesh* mesh, T
         ht[i] = DevTexture{mesh->textures[i].texels, mesh->textures[i].width, mesh->textures[i].height};
     out->count = (uint32_t)ntris;
     VCT_TRY(ensure(ctx->soup_pos, 36u * (ntris ? ntris : 1)));
-    VCT_TRY(ensure(ctx->soup_nrm, 36u * (ntris ? ntris : 1)));
+    if (normals) VCT_TRY(ensure(ctx->soup_nrm, 36u * (ntris ? ntris : 1)));
     VCT_TRY(ensure(ctx->soup_mat, 4u * (ntris ? ntris : 1)));
-    VCT_TRY(ensure(ctx->soup_uv, 24u * (ntris ? ntris : 1)));
+    if (sampled) VCT_TRY(ensure(ctx->soup_uv, 24u * (ntris ? ntris : 1)));
     out->pos = (const float*)ctx->soup_pos.ptr;
-    out->nrm = (const float*)ctx->soup_nrm.ptr;
+    out->nrm = normals ? (const float*)ctx->soup_nrm.ptr : nullptr;
     out->mat = (const uint32_t*)ctx->soup_mat.ptr;
-    out->uv = (const float*)ctx->soup_uv.ptr;
+    out->uv = sampled ? (const float*)ctx->soup_uv.ptr : nullptr;
     out->tex = nullptr;
     out->tex_count = 0;
     if (ntris == 0) return VCT_OK;
@@ -285,8 +291,8 @@ vct_status run_vertex_stage(vct_ctx* ctx, hipStream_t s, const vct_mesh* mesh, T
     uint32_t blocks = (uint32_t)((ntris + threads - 1) / threads);
     hipLaunchKernelGGL(k_vertex_stage, dim3(blocks), dim3(threads), 0, s, mesh->positions, mesh->normals,
                        mesh->texcoords, mesh->indices, mesh->node_matrices, (const DevPrim*)ctx->prims.ptr, n,
-                       (uint32_t)ntris, (float*)ctx->soup_pos.ptr, (float*)ctx->soup_nrm.ptr,
-                       (uint32_t*)ctx->soup_mat.ptr, (float*)ctx->soup_uv.ptr);
+                       (uint32_t)ntris, (float*)ctx->soup_pos.ptr, normals ? (float*)ctx->soup_nrm.ptr : nullptr,
+                       (uint32_t*)ctx->soup_mat.ptr, ntex ? (float*)ctx->soup_uv.ptr : nullptr);
     VCT_HIP(hipGetLastError());
     return VCT_OK;
 }

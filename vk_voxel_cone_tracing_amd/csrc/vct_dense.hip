@@ -10,13 +10,13 @@
 // carries a one-texel zero border so the trilinear footprint never needs a
 // bounds test inside the grid. Texels are RGBA8 or RGBA32F.
 #include <hip/hip_runtime.h>
-#include <hipcub/hipcub.hpp>
 
 #include <cmath>
 #include <new>
 
 #include "vct_dense.hpp"
 #include "vct_dense_mip.hpp"
+#include "vct_expand.hpp"
 #include "vct_internal.hpp"
 #include "vct_raster.hpp"
 #include "vct_texel.hpp"
@@ -39,16 +39,6 @@ vct_status dense_alloc(vct_dense* g)
     return ensure(g->data, total * g->texel_bytes);
 }
 
-__global__ void k_dense_translate(const float* __restrict__ pos, uint32_t n9, float mx, float my, float mz,
-                                  float* __restrict__ out)
-{
-#pragma clang fp contract(off)
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n9) return;
-    const uint32_t k = i % 3u;
-    out[i] = pos[i] - (k == 0 ? mx : (k == 1 ? my : mz));
-}
-
 struct DenseRaster {
     float vs;
     int lo[3], hi[3];
@@ -56,24 +46,36 @@ struct DenseRaster {
     int res;
 };
 
-__global__ void k_dense_count(const float* __restrict__ tpos, uint32_t ntris, DenseRaster R,
-                              unsigned long long* __restrict__ counts)
+// A triangle in grid coordinates (written to tpos) and its item count, scanned
+// within the workgroup's 256 triangles.
+__global__ __launch_bounds__(kExpandBlock) void k_dense_count(const float* __restrict__ pos, uint32_t ntris, float mx,
+                                                              float my, float mz, DenseRaster R,
+                                                              float* __restrict__ tpos,
+                                                              unsigned long long* __restrict__ in_block,
+                                                              unsigned long long* __restrict__ block_sums)
 {
-    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= ntris) return;
-    float p[9];
-    for (int k = 0; k < 9; ++k) p[k] = tpos[9u * t + k];
-    TriSetup s;
+#pragma clang fp contract(off)
+    const uint32_t t = blockIdx.x * kExpandBlock + threadIdx.x;
     unsigned long long n = 0;
-    if (tri_setup(p, R.vs, R.lo, R.hi, s)) n = (unsigned long long)s.nu * s.nv * (unsigned long long)R.samples;
-    counts[t] = n;
+    if (t < ntris) {
+        float p[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            p[k] = pos[9u * t + k] - (k % 3 == 0 ? mx : (k % 3 == 1 ? my : mz));
+            tpos[9u * t + k] = p[k];
+        }
+        TriSetup s;
+        if (tri_setup(p, R.vs, R.lo, R.hi, s)) n = (unsigned long long)s.nu * s.nv * (unsigned long long)R.samples;
+    }
+    const unsigned long long below = expand_block(n, &block_sums[blockIdx.x]);
+    in_block[blockIdx.x * kExpandBlock + threadIdx.x] = below;
 }
 
-__global__ void k_dense_total(const unsigned long long* __restrict__ counts,
-                              const unsigned long long* __restrict__ offsets, uint32_t n,
-                              unsigned long long* __restrict__ total)
+__global__ __launch_bounds__(1024) void k_dense_total(unsigned long long* __restrict__ blocks, uint32_t nblocks,
+                                                      unsigned long long* __restrict__ total)
 {
-    total[0] = n ? offsets[n - 1] + counts[n - 1] : 0ull;
+    const unsigned long long all = expand_scan(blocks, nblocks);
+    if (threadIdx.x == 0) total[0] = all;
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v)
@@ -84,28 +86,26 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v)
 
 // Every covered sample proposes its triangle for its voxel; the smallest
 // triangle index (the first fragment in rasterization order) wins.
-__global__ __launch_bounds__(256) void k_dense_raster(const float* __restrict__ tpos,
-                                                      const unsigned long long* __restrict__ offsets, uint32_t ntris,
+__global__ __launch_bounds__(256) void k_dense_raster(const float* __restrict__ tpos, Expansion E, uint32_t ntris,
                                                       const unsigned long long* __restrict__ total, DenseRaster R,
                                                       uint32_t* __restrict__ winner)
 {
 #pragma clang fp contract(off)
     const unsigned long long n = total[0];
     const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
-    for (unsigned long long wi = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; wi < n; wi += stride) {
-        uint32_t lo = 0, hi = ntris;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (offsets[mid] <= wi) lo = mid; else hi = mid;
-        }
-        const uint32_t t = lo;
+    // whole waves: the search takes all 64 lanes
+    for (unsigned long long first = (unsigned long long)blockIdx.x * blockDim.x + (threadIdx.x & ~63u); first < n;
+         first += stride) {
+        const uint32_t t = wave_triangle(E, ntris, first, n - 1ull);
+        const unsigned long long wi = first + (threadIdx.x & 63u);
+        if (wi >= n) continue;
         float p[9];
         for (int k = 0; k < 9; ++k) p[k] = tpos[9u * t + k];
         TriSetup s;
         if (!tri_setup(p, R.vs, R.lo, R.hi, s)) continue;
         float fp[3];
         double lam[3];
-        if (!tri_sample(p, s, R.vs, R.samples, (uint32_t)(wi - offsets[t]), fp, lam)) continue;
+        if (!tri_sample(p, s, R.vs, R.samples, (uint32_t)(wi - E(t)), fp, lam)) continue;
         int ic[3];
         bool inside = true;
         for (int k = 0; k < 3; ++k) {
@@ -118,20 +118,41 @@ __global__ __launch_bounds__(256) void k_dense_raster(const float* __restrict__ 
     }
 }
 
-template <bool kF32>
-__global__ void k_dense_resolve(const uint32_t* __restrict__ winner, const uint32_t* __restrict__ mat,
-                                const vct_gltf_material* __restrict__ mats, int res, void* __restrict__ level0)
+// The winners' colours into level 0; every winner is returned to empty for the
+// next voxelization. A thread takes kPer consecutive voxels of a row (4 of a
+// row of at least 4: one 16-byte read, and nearly all are empty). Bound by the
+// read of the winners. 256^3: 51 us with one voxel a thread and divisions by
+// the resolution, 32 us so; the fill of the winners before each voxelization
+// (18 us) is gone.
+template <bool kF32, int kPer>
+__global__ __launch_bounds__(256) void k_dense_resolve(uint32_t* __restrict__ winner, const uint32_t* __restrict__ mat,
+                                                       const vct_gltf_material* __restrict__ mats, int log2_res,
+                                                       void* __restrict__ level0)
 {
-    const size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= (size_t)res * res * res) return;
-    const uint32_t t = winner[v];
-    if (t == 0xffffffffu) return;
-    const int x = (int)(v % res), y = (int)((v / res) % res), z = (int)(v / ((size_t)res * res));
+    const uint32_t v = (blockIdx.x * 256u + threadIdx.x) * kPer, res = 1u << log2_res;  // res <= 1024
+    if (v >> (3 * log2_res)) return;
+    uint32_t t[kPer];
+    if (kPer == 4) {
+        const uint4 q = *(const uint4*)(winner + v);
+        if ((q.x & q.y & q.z & q.w) == 0xffffffffu) return;
+        t[0] = q.x;
+        t[1 % kPer] = q.y;
+        t[2 % kPer] = q.z;
+        t[3 % kPer] = q.w;
+    } else {
+        t[0] = winner[v];
+    }
+    const uint32_t x = v & (res - 1u), y = (v >> log2_res) & (res - 1u), z = v >> (2 * log2_res);
     const size_t D = (size_t)res + 2;
     const size_t i = ((size_t)(z + 1) * D + (size_t)(y + 1)) * D + (size_t)(x + 1);
-    const float* bc = mats[mat[t]].base_color_factor;
-    if (kF32) ((float4*)level0)[i] = make_float4(bc[0], bc[1], bc[2], 1.0f);
-    else ((uint32_t*)level0)[i] = pack_unorm(f4{bc[0], bc[1], bc[2], 1.0f});
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        if (t[k] == 0xffffffffu) continue;
+        winner[v + k] = 0xffffffffu;
+        const float* bc = mats[mat[t[k]]].base_color_factor;
+        if (kF32) ((float4*)level0)[i + k] = make_float4(bc[0], bc[1], bc[2], 1.0f);
+        else ((uint32_t*)level0)[i + k] = pack_unorm(f4{bc[0], bc[1], bc[2], 1.0f});
+    }
 }
 
 // radianceDownSample.comp:95-139 over the whole grid. Level 1 (kFirst): one
@@ -267,13 +288,10 @@ vct_status vct_dense_voxelize(vct_dense* g, vct_stream stream, const vct_mesh* m
     hipStream_t s = (hipStream_t)stream;
     vct_ctx* c = g->scratch;
     TriSoup soup;
-    VCT_TRY(run_vertex_stage(c, s, mesh, &soup, TextureUse::kRefuse));
+    VCT_TRY(run_vertex_stage(c, s, mesh, &soup, TextureUse::kRefuse, false));
     if (!soup.count) return VCT_OK;
-    const uint32_t n9 = soup.count * 9u;
-    VCT_TRY(ensure(c->rec_val, 4u * (size_t)n9));
+    VCT_TRY(ensure(c->rec_val, 36u * (size_t)soup.count));
     float* tpos = (float*)c->rec_val.ptr;
-    hipLaunchKernelGGL(k_dense_translate, dim3((n9 + 255) / 256), dim3(256), 0, s, soup.pos, n9, g->desc.grid_min[0],
-                       g->desc.grid_min[1], g->desc.grid_min[2], tpos);
     DenseRaster R;
     R.vs = g->desc.extent / (float)g->res;
     for (int k = 0; k < 3; ++k) {
@@ -282,31 +300,33 @@ vct_status vct_dense_voxelize(vct_dense* g, vct_stream stream, const vct_mesh* m
     }
     R.samples = (int)g->desc.raster_samples;
     R.res = g->res;
-    VCT_TRY(ensure(c->counts, 8u * (size_t)soup.count));
-    VCT_TRY(ensure(c->offsets, 8u * (size_t)soup.count));
+    const uint32_t nblocks = (soup.count + kExpandBlock - 1u) / kExpandBlock;
+    VCT_TRY(ensure(c->counts, 8u * (size_t)nblocks * kExpandBlock));
+    VCT_TRY(ensure(c->offsets, 8u * (size_t)nblocks));
     VCT_TRY(ensure(c->totals, 64));
-    hipLaunchKernelGGL(k_dense_count, dim3((soup.count + 255) / 256), dim3(256), 0, s, tpos, soup.count, R,
-                       (unsigned long long*)c->counts.ptr);
-    size_t tmp = 0;
-    VCT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, (unsigned long long*)c->counts.ptr,
-                                             (unsigned long long*)c->offsets.ptr, (int)soup.count, s));
-    VCT_TRY(ensure(c->scan_tmp, tmp));
-    VCT_HIP(hipcub::DeviceScan::ExclusiveSum(c->scan_tmp.ptr, tmp, (unsigned long long*)c->counts.ptr,
-                                             (unsigned long long*)c->offsets.ptr, (int)soup.count, s));
-    hipLaunchKernelGGL(k_dense_total, dim3(1), dim3(1), 0, s, (const unsigned long long*)c->counts.ptr,
-                       (const unsigned long long*)c->offsets.ptr, soup.count, (unsigned long long*)c->totals.ptr);
     const size_t nv = (size_t)g->res * g->res * g->res;
+    const bool fresh = !g->winner.ptr;
     VCT_TRY(ensure(g->winner, 4u * nv));
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, s, (uint32_t*)g->winner.ptr, nv,
-                       0xffffffffu);
-    hipLaunchKernelGGL(k_dense_raster, dim3(8192), dim3(256), 0, s, tpos, (const unsigned long long*)c->offsets.ptr,
-                       soup.count, (const unsigned long long*)c->totals.ptr, R, (uint32_t*)g->winner.ptr);
-    if (g->texel_bytes == 16)
-        hipLaunchKernelGGL(k_dense_resolve<true>, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, s,
-                           (const uint32_t*)g->winner.ptr, soup.mat, mesh->materials, g->res, g->data.ptr);
-    else
-        hipLaunchKernelGGL(k_dense_resolve<false>, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, s,
-                           (const uint32_t*)g->winner.ptr, soup.mat, mesh->materials, g->res, g->data.ptr);
+    if (fresh)  // every voxelization leaves the winners empty
+        hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, s, (uint32_t*)g->winner.ptr,
+                           nv, 0xffffffffu);
+    const Expansion E{(const unsigned long long*)c->counts.ptr, (const unsigned long long*)c->offsets.ptr};
+    auto* total = (unsigned long long*)c->totals.ptr;
+    hipLaunchKernelGGL(k_dense_count, dim3(nblocks), dim3(kExpandBlock), 0, s, soup.pos, soup.count,
+                       g->desc.grid_min[0], g->desc.grid_min[1], g->desc.grid_min[2], R, tpos,
+                       (unsigned long long*)c->counts.ptr, (unsigned long long*)c->offsets.ptr);
+    hipLaunchKernelGGL(k_dense_total, dim3(1), dim3(1024), 0, s, (unsigned long long*)c->offsets.ptr, nblocks, total);
+    hipLaunchKernelGGL(k_dense_raster, dim3(8192), dim3(256), 0, s, (const float*)tpos, E, soup.count,
+                       (const unsigned long long*)total, R, (uint32_t*)g->winner.ptr);
+    int log2_res = 0;
+    while ((1 << log2_res) < g->res) ++log2_res;
+    auto resolve = [&](auto kernel, size_t per) {
+        const size_t threads = (nv + per - 1) / per;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s,
+                           (uint32_t*)g->winner.ptr, soup.mat, mesh->materials, log2_res, g->data.ptr);
+    };
+    if (g->texel_bytes == 16) g->res >= 4 ? resolve(k_dense_resolve<true, 4>, 4) : resolve(k_dense_resolve<true, 1>, 1);
+    else g->res >= 4 ? resolve(k_dense_resolve<false, 4>, 4) : resolve(k_dense_resolve<false, 1>, 1);
     VCT_HIP(hipGetLastError());
     return VCT_OK;
 }

@@ -17,19 +17,19 @@ constexpr uint32_t kExpandBlock = 256;  // triangles per block: the counting ker
 // Where each triangle's items begin: triangle t's are numbered from
 // block[t / 256] + in_block[t].
 struct Expansion {
-    const uint32_t* in_block;
+    const unsigned long long* in_block;
     const unsigned long long* block;
 
     __device__ __forceinline__ unsigned long long operator()(uint32_t t) const
     {
-        return block[t / kExpandBlock] + (unsigned long long)in_block[t];
+        return block[t / kExpandBlock] + in_block[t];
     }
 };
 
 // Called by every thread of a 256-thread workgroup with its triangle's item
 // count (0 past the last triangle): returns the sum of the lower threads'
-// counts and leaves the workgroup's sum in *block_sum. A block's items number
-// less than 2^32: a triangle has at most 4 x 4098^2 of them.
+// counts and leaves the workgroup's sum in *block_sum. Sums are 64 bits wide: 256
+// triangles of millions of samples each pass 2^32.
 __device__ __forceinline__ unsigned long long expand_block(unsigned long long count, unsigned long long* block_sum)
 {
     __shared__ unsigned long long wave_sum[kExpandBlock / 64];

@@ -55,9 +55,9 @@ struct DevTexture;
 // World-space triangle soup produced by the vertex stage.
 struct TriSoup {
     const float* pos;     // 9 floats per triangle
-    const float* nrm;     // 9 floats per triangle
+    const float* nrm;     // 9 floats per triangle (null unless asked for)
     const uint32_t* mat;  // material index per triangle
-    const float* uv;      // 6 floats per triangle (zero without texcoords)
+    const float* uv;      // 6 floats per triangle (null without a texture table)
     const DevTexture* tex;  // the mesh's textures on the device (null without a table)
     uint32_t tex_count;
     uint32_t count;
@@ -191,9 +191,10 @@ __device__ __forceinline__ unsigned xcd_remap(unsigned b, unsigned n)
 // texture coordinates and the mesh's texture table on the device. A draw
 // list whose materials reference a base-colour, emissive or occlusion
 // texture is refused (VCT_ERR_UNSUPPORTED) with TextureUse::kRefuse; with
-// kSample every such index must name one of the mesh's textures.
+// kSample every such index must name one of the mesh's textures. Without
+// `normals` the soup holds none.
 vct_status run_vertex_stage(vct_ctx* ctx, hipStream_t s, const vct_mesh* mesh, TriSoup* out,
-                            TextureUse use = TextureUse::kSample);
+                            TextureUse use = TextureUse::kSample, bool normals = true);
 
 // The base-colour, emissive and occlusion texture indices of every material
 // of a device material table (3 per material), read back to the host.

@@ -106,7 +106,7 @@ struct LevelSet {
 // block's sum. With k_total this is the whole scan, 10 us in two launches (a
 // library scan of the counts: 18 us in four).
 __global__ __launch_bounds__(kExpandBlock) void k_count(const float* __restrict__ pos, uint32_t ntris, LevelSet S,
-                                                        uint32_t* __restrict__ in_block,
+                                                        unsigned long long* __restrict__ in_block,
                                                         unsigned long long* __restrict__ block_sums)
 {
     const uint32_t t = blockIdx.x * kExpandBlock + threadIdx.x, slot = blockIdx.y;
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(kExpandBlock) void k_count(const float* __restrict_
     }
     const uint32_t b = slot * gridDim.x + blockIdx.x;
     const unsigned long long below = expand_block(n, &block_sums[b]);
-    in_block[(size_t)b * kExpandBlock + threadIdx.x] = (uint32_t)below;
+    in_block[(size_t)b * kExpandBlock + threadIdx.x] = below;
 }
 
 // The work items of the slots are numbered consecutively, each slot starting
@@ -581,16 +581,16 @@ static vct_status expand(vct_ctx* c, hipStream_t s, const TriSoup& soup, const L
     const size_t n = (size_t)nblocks * (size_t)S.n;
     if ((size_t)soup.count * (size_t)S.n > 0x7fffffffull)
         return fail(VCT_ERR_CAPACITY, "%zu triangle-level pairs exceed 2^31", (size_t)soup.count * (size_t)S.n);
-    VCT_TRY(ensure(c->counts, 4u * (n ? n : 1) * kExpandBlock));
+    VCT_TRY(ensure(c->counts, 8u * (n ? n : 1) * kExpandBlock));
     VCT_TRY(ensure(c->offsets, 8u * (n ? n : 1)));
     VCT_TRY(ensure(c->totals, 8u * kTotWords));
     if (n)
         hipLaunchKernelGGL(k_count, dim3(nblocks, (unsigned)S.n), dim3(kExpandBlock), 0, s, soup.pos, soup.count, S,
-                           (uint32_t*)c->counts.ptr, (unsigned long long*)c->offsets.ptr);
+                           (unsigned long long*)c->counts.ptr, (unsigned long long*)c->offsets.ptr);
     hipLaunchKernelGGL(k_total, dim3(1), dim3(1024), 0, s, (unsigned long long*)c->offsets.ptr, nblocks, S.n,
                        (unsigned long long*)c->totals.ptr);
     VCT_HIP(hipGetLastError());
-    *E = {(const uint32_t*)c->counts.ptr, (const unsigned long long*)c->offsets.ptr};
+    *E = {(const unsigned long long*)c->counts.ptr, (const unsigned long long*)c->offsets.ptr};
     return VCT_OK;
 }
 
@@ -601,7 +601,7 @@ static vct_status voxelize_levels(vct_ctx* c, hipStream_t s, const vct_mesh* mes
     LevelSet S;
     VCT_TRY(make_level_set(c, descs, count, &S));
     TriSoup soup;
-    VCT_TRY(run_vertex_stage(c, s, mesh, &soup));
+    VCT_TRY(run_vertex_stage(c, s, mesh, &soup, TextureUse::kSample, false));
     if (!soup.count) return VCT_OK;
     Expansion E;
     VCT_TRY(expand(c, s, soup, S, &E));
