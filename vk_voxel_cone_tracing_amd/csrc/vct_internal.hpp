@@ -69,7 +69,6 @@ enum class TextureUse { kSample, kRefuse, kIgnore };
 struct SvoState {
     DeviceBuffer frags;      // uvec2 per fragment
     DeviceBuffer pool;       // uvec2 per node
-    DeviceBuffer counters;   // small device counters
     uint32_t nfrag = 0;
     uint32_t level = 0;
     uint32_t pool_nodes = 0; // capacity

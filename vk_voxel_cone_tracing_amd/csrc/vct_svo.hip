@@ -7,11 +7,11 @@
 //  * every covered raster sample gets its slot from an exclusive scan over the
 //    (triangle, cell, sample) work items, i.e. rasterization order;
 //  * child blocks are handed to the flagged nodes of a level in pool-index
-//    order with a wavefront ballot/popcount prefix scan (three passes: wave
-//    counts, block offsets, assignment), which is the reference's outcome
-//    when invocations run in index order;
+//    order, which is the reference's outcome when invocations run in index
+//    order: with the fragments sorted by leaf path, a node's place follows
+//    from its rank among the distinct path prefixes of its depth;
 //  * the order-dependent leaf running average is applied per leaf in
-//    fragment order after a radix sort keyed by (leaf, fragment).
+//    fragment order (the sort by path is stable).
 // The node pool is therefore a pure function of the fragment list.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -19,6 +19,7 @@
 #include <cmath>
 #include <vector>
 
+#include "vct_expand.hpp"
 #include "vct_internal.hpp"
 #include "vct_raster.hpp"
 #include "vct_shadow.hpp"
@@ -219,114 +220,158 @@ __device__ __forceinline__ uint32_t walk(const uint2* __restrict__ pool, uint32_
     return idx;
 }
 
-// octreeNodeFlag.comp: mark the deepest existing node of every fragment.
-// The pass at `depth` would walk from the root along the previous pass's
-// path and one step further (the node a fragment reached then was flagged,
-// so it has children now): node_of keeps each fragment's node between passes
-// and the pass takes that one step. The child slot at depth d is bit
-// L - 1 - d of the position (z | x << 1 | y << 2, as in walk()); a coordinate
-// of 2^L takes walk()'s path for 2^L - 1.
-__global__ __launch_bounds__(256) void k_svo_flag(uint2* __restrict__ pool, const uint2* __restrict__ frags,
-                                                  uint32_t nfrag, uint32_t L, uint32_t depth, bool half,
-                                                  uint32_t* __restrict__ node_of)
+// The tree is built from the fragments sorted by their leaf's path: the child
+// slots from the root down (z | x << 1 | y << 2 per depth, as in walk()), most
+// significant first. octreeNodeAlloc hands out child blocks in pool order, and
+// the nodes of a depth lie in the order of their parents' blocks, so by
+// induction the pool order of a depth's nodes is the order of their paths. The
+// nodes that some fragment reaches at depth e are the distinct prefixes of
+// e + 1 slots; one's rank among them, and the number G_e of such nodes above
+// depth e, give its child block (G_e + rank + 1) << 3, and its parent's block
+// and its last slot give its index. One sort, one counting pass and one
+// writing pass build every depth, with one read-back of the sizes, where a
+// flag pass over all fragments (with atomics), an allocation (count, scan,
+// assign) and a read-back per depth were needed. 2^9 per axis, 1M triangles:
+// nine flag passes 880 us, nine allocations 190 us, leaf keys and averages 156
+// us and a sort of 50-bit keys 290 us, now keys 16 us, a sort of 27-bit keys
+// with their colours 245 us, counts 19 us and nodes with averages 82 us. Bound
+// by the sort's passes over memory.
+
+// A coordinate of 2^L takes walk()'s path for 2^L - 1.
+template <typename Key>
+__global__ __launch_bounds__(256) void k_svo_keys(const uint2* __restrict__ frags, uint32_t nfrag, uint32_t L,
+                                                  bool half, Key* __restrict__ keys, uint32_t* __restrict__ colors)
 {
     const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nfrag) return;
+    const uint2 v = frags[f];
     uint32_t p[3];
-    frag_pos(frags[f], half, p);
-    const uint32_t top = (1u << L) - 1u, b = L - 1u - depth;
-    const uint32_t x = min(p[0], top), y = min(p[1], top), z = min(p[2], top);
-    const uint32_t slot = ((z >> b) & 1u) | (((x >> b) & 1u) << 1) | (((y >> b) & 1u) << 2);
-    uint32_t idx = slot;
-    if (depth > 0) {
-        const uint32_t parent = node_of[f];
-        const uint32_t cur = pool[parent].x & 0x7fffffffu;
-        idx = cur ? cur + slot : parent;  // walk() stops at a node without children
-    }
-    node_of[f] = idx;
-    // Setting a set bit changes nothing, so the pool ends the same when the
-    // lanes of a wave that reach one node leave it to one of them, and when a
-    // flag already visible is not set again. Near the root the fragments of a
-    // wave reach a few nodes (nearly all fragments reach one node at the
-    // first depth), and atomics on one address serialize: up to four of a
-    // wave's nodes are flagged by one lane each, the rest lane by lane.
-    const uint32_t lane = __lane_id();
-    bool todo = true;
+    frag_pos(v, half, p);
+    const uint32_t top = (1u << L) - 1u;
+    auto spread = [](uint32_t c) -> Key {  // bit b to bit 3b
+        uint32_t r = c & 1023u;
+        r = (r | (r << 16)) & 0x030000ffu;
+        r = (r | (r << 8)) & 0x0300f00fu;
+        r = (r | (r << 4)) & 0x030c30c3u;
+        r = (r | (r << 2)) & 0x09249249u;
+        Key k = r;
+        if (sizeof(Key) == 8) k |= (Key)(c >> 10) << (sizeof(Key) == 8 ? 30 : 0);
+        return k;
+    };
+    keys[f] = spread(min(p[2], top)) | (spread(min(p[0], top)) << 1) | (spread(min(p[1], top)) << 2);
+    colors[f] = v.y & 0x0fffffffu;
+}
+
+constexpr uint32_t kSvoMaxDepth = 11;  // octree levels
+constexpr uint32_t kNodeKeys = 1024;   // sorted fragments per workgroup, 256 per wave in four chunks
+
+// The first depth at which sorted fragment i reaches another node than
+// fragment i - 1 (L where both reach one leaf; L also past the last fragment).
+template <typename Key>
+__device__ __forceinline__ uint32_t first_new_depth(const Key* __restrict__ keys, uint32_t i, uint32_t n, uint32_t L,
+                                                    Key& key)
+{
+    key = 0;
+    if (i >= n) return L;
+    key = keys[i];
+    if (i == 0) return 0u;
+    const unsigned long long d = (unsigned long long)(key ^ keys[i - 1]);
+    return d ? L - 1u - (63u - (uint32_t)__clzll((long long)d)) / 3u : L;
+}
+
+// New nodes per depth of every workgroup's fragments: counts[depth][workgroup].
+template <typename Key>
+__global__ __launch_bounds__(256) void k_svo_node_count(const Key* __restrict__ keys, uint32_t n, uint32_t L,
+                                                        unsigned long long* __restrict__ counts)
+{
+    __shared__ uint32_t s_count[4][kSvoMaxDepth];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t first = blockIdx.x * kNodeKeys + wave * (kNodeKeys / 4u);
+    uint32_t mine[kSvoMaxDepth] = {};
 #pragma unroll
-    for (int round = 0; round < 4; ++round) {
-        const unsigned long long left = __ballot(todo);
-        if (left == 0ull) break;
-        const int leader = __ffsll((long long)left) - 1;
-        const uint32_t node = __builtin_amdgcn_readlane(idx, leader);
-        if (todo && idx == node) {
-            todo = false;
-            if ((int)lane == leader && !(pool[idx].x & 0x80000000u)) atomicOr(&pool[idx].x, 0x80000000u);
+    for (uint32_t c = 0; c < kNodeKeys / 256u; ++c) {
+        Key key;
+        const uint32_t f = first_new_depth(keys, first + c * 64u + lane, n, L, key);
+#pragma unroll
+        for (uint32_t e = 0; e < kSvoMaxDepth; ++e)
+            if (e < L) mine[e] += (uint32_t)__popcll(__ballot(f <= e));
+    }
+    if (lane == 0u)
+        for (uint32_t e = 0; e < L; ++e) s_count[wave][e] = mine[e];
+    __syncthreads();
+    if (threadIdx.x < L)
+        counts[(size_t)threadIdx.x * gridDim.x + blockIdx.x] =
+            (unsigned long long)s_count[0][threadIdx.x] + s_count[1][threadIdx.x] + s_count[2][threadIdx.x] +
+            s_count[3][threadIdx.x];
+}
+
+// One workgroup per depth: the prefix of its counts over the workgroups, and
+// the depth's number of nodes.
+__global__ __launch_bounds__(1024) void k_svo_node_scan(unsigned long long* __restrict__ counts, uint32_t nblocks,
+                                                        unsigned long long* __restrict__ totals)
+{
+    const unsigned long long all = expand_scan(counts + (size_t)blockIdx.x * nblocks, nblocks);
+    if (threadIdx.x == 0) totals[blockIdx.x] = all;
+}
+
+// Every node some fragment reaches, written by the first of its fragments (the
+// pool is zero before), and each leaf's running average over its fragments in
+// fragment order (octreeNodeLeafWrite.comp; the sort is stable).
+template <typename Key>
+__global__ __launch_bounds__(256) void k_svo_nodes(const Key* __restrict__ keys, const uint32_t* __restrict__ colors,
+                                                   uint32_t n, uint32_t L,
+                                                   const unsigned long long* __restrict__ counts,
+                                                   const unsigned long long* __restrict__ totals,
+                                                   uint2* __restrict__ pool)
+{
+    __shared__ uint32_t s_count[4][kSvoMaxDepth];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t first = blockIdx.x * kNodeKeys + wave * (kNodeKeys / 4u);
+    constexpr uint32_t kChunks = kNodeKeys / 256u;
+    uint32_t f[kChunks], rank[kSvoMaxDepth] = {};
+    Key key[kChunks];
+#pragma unroll
+    for (uint32_t c = 0; c < kChunks; ++c) {
+        f[c] = first_new_depth(keys, first + c * 64u + lane, n, L, key[c]);
+#pragma unroll
+        for (uint32_t e = 0; e < kSvoMaxDepth; ++e)
+            if (e < L) rank[e] += (uint32_t)__popcll(__ballot(f[c] <= e));
+    }
+    if (lane == 0u)
+        for (uint32_t e = 0; e < L; ++e) s_count[wave][e] = rank[e];
+    __syncthreads();
+    // nodes of each depth begun before this wave's first fragment
+#pragma unroll
+    for (uint32_t e = 0; e < kSvoMaxDepth; ++e)
+        if (e < L) {
+            rank[e] = (uint32_t)counts[(size_t)e * gridDim.x + blockIdx.x];
+            for (uint32_t w = 0; w < wave; ++w) rank[e] += s_count[w][e];
+        }
+    const unsigned long long upto = ~0ull >> (63u - lane);  // this lane and those below
+#pragma unroll
+    for (uint32_t c = 0; c < kChunks; ++c) {
+        uint32_t block = 0;   // the child block that depth e's node lies in
+        uint32_t above = 0;   // G_e
+#pragma unroll
+        for (uint32_t e = 0; e < kSvoMaxDepth; ++e) {
+            if (e >= L) continue;
+            const unsigned long long m = __ballot(f[c] <= e);
+            const uint32_t child = (above + rank[e] + (uint32_t)__popcll(m & upto)) << 3;
+            const uint32_t idx = block + ((uint32_t)(key[c] >> (3u * (L - 1u - e))) & 7u);
+            if (f[c] <= e) {
+                uint2 node = make_uint2(child | 0x80000000u, 0u);
+                if (e == L - 1u) {
+                    node.x = 0x80000000u;
+                    for (uint32_t i = first + c * 64u + lane; i < n && keys[i] == key[c]; ++i)
+                        node.y = rgba8_avg(node.y, unpack_raw(colors[i]));
+                }
+                pool[idx] = node;
+            }
+            block = child;
+            above += (uint32_t)totals[e];
+            rank[e] += (uint32_t)__popcll(m);
         }
     }
-    if (todo && !(pool[idx].x & 0x80000000u)) atomicOr(&pool[idx].x, 0x80000000u);
-}
-
-// octreeNodeAlloc.comp with ordered allocation. Pass 1: per-wave flagged counts.
-__global__ __launch_bounds__(256) void k_svo_alloc_count(const uint2* __restrict__ pool, uint32_t begin, uint32_t num,
-                                                         uint32_t* __restrict__ wave_counts)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool flagged = i < num && (pool[begin + i].x & 0x80000000u);
-    const unsigned long long ballot = __ballot(flagged);
-    if ((threadIdx.x & 63) == 0) wave_counts[i >> 6] = (uint32_t)__popcll(ballot);
-}
-
-// Pass 3: rank = wave offset + popcount of lower lanes; child block
-// (base + rank + 1) << 3 with the subdivide flag kept.
-__global__ __launch_bounds__(256) void k_svo_alloc_assign(uint2* __restrict__ pool, uint32_t begin, uint32_t num,
-                                                          const uint32_t* __restrict__ wave_offsets, uint32_t base)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool flagged = i < num && (pool[begin + i].x & 0x80000000u);
-    const unsigned long long ballot = __ballot(flagged);
-    if (!flagged) return;
-    const uint32_t lane = threadIdx.x & 63;
-    const unsigned long long lower = lane ? (ballot & (~0ull >> (64 - lane))) : 0ull;
-    const uint32_t rank = wave_offsets[i >> 6] + (uint32_t)__popcll(lower);
-    pool[begin + i] = make_uint2(((base + rank + 1u) << 3u) | 0x80000000u, 0u);
-}
-
-// octreeNodeModifyArg.comp: the child blocks handed out so far, on the device
-// (the last wave's offset plus its count), read back once per level.
-__global__ void k_svo_advance(const uint32_t* __restrict__ wave_offsets, const uint32_t* __restrict__ wave_counts,
-                              uint32_t waves, uint32_t* __restrict__ counter)
-{
-    counter[0] += wave_offsets[waves - 1] + wave_counts[waves - 1];
-}
-
-// octreeNodeLeafWrite.comp, ordered: one key (leaf << fbits | fragment) per
-// fragment that reaches a leaf; fragments that do not take `none`, above
-// every such key, and sort last.
-__global__ __launch_bounds__(256) void k_svo_leaf_keys(const uint2* __restrict__ pool, const uint2* __restrict__ frags,
-                                                       uint32_t nfrag, uint32_t R, bool half, uint32_t fbits,
-                                                       unsigned long long none, unsigned long long* __restrict__ keys)
-{
-    const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nfrag) return;
-    uint32_t p[3], r;
-    frag_pos(frags[f], half, p);
-    const uint32_t idx = walk(pool, p, R, 1u, r);
-    keys[f] = r == 1u ? (((unsigned long long)idx << fbits) | f) : none;
-}
-
-__global__ __launch_bounds__(256) void k_svo_leaf_apply(uint2* __restrict__ pool, const uint2* __restrict__ frags,
-                                                        const unsigned long long* __restrict__ keys, uint32_t n,
-                                                        uint32_t fbits, unsigned long long none)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || keys[i] == none) return;
-    const unsigned long long leaf = keys[i] >> fbits;
-    if (i > 0 && (keys[i - 1] >> fbits) == leaf) return;
-    const unsigned long long fmask = (1ull << fbits) - 1ull;
-    uint32_t t = pool[leaf].y;
-    for (uint32_t j = i; j < n && keys[j] != none && (keys[j] >> fbits) == leaf; ++j)
-        t = rgba8_avg(t, unpack_raw(frags[(uint32_t)(keys[j] & fmask)].y & 0x0fffffffu));
-    pool[leaf].y = t;
 }
 
 // octreeNodeMipmapWrite.comp evaluated per node: every flagged node of the
@@ -393,6 +438,43 @@ static LightParams make_light(const vct_shadow_map* shadow, const vct_directiona
 static unsigned blocks_for(uint64_t n, unsigned threads = 256)
 {
     return (unsigned)((n + threads - 1) / threads);
+}
+
+// The fragments sorted by path (keys in rec_key[1], colours in rec_idx[1]) and
+// the new nodes per depth: totals[depth], scanned per workgroup in counts.
+template <typename Key>
+static vct_status svo_sort(vct_ctx* c, hipStream_t s, const uint2* frags, uint32_t nfrag, uint32_t L, bool half)
+{
+    const uint32_t nblocks = blocks_for(nfrag, kNodeKeys);
+    for (int b = 0; b < 2; ++b) {
+        VCT_TRY(ensure(c->rec_key[b], sizeof(Key) * (size_t)nfrag));
+        VCT_TRY(ensure(c->rec_idx[b], 4u * (size_t)nfrag));
+    }
+    VCT_TRY(ensure(c->counts, 8u * (size_t)L * nblocks));
+    VCT_TRY(ensure(c->totals, 8u * kSvoMaxDepth));
+    Key* k0 = (Key*)c->rec_key[0].ptr;
+    Key* k1 = (Key*)c->rec_key[1].ptr;
+    uint32_t* v0 = (uint32_t*)c->rec_idx[0].ptr;
+    uint32_t* v1 = (uint32_t*)c->rec_idx[1].ptr;
+    hipLaunchKernelGGL(k_svo_keys<Key>, dim3(blocks_for(nfrag)), dim3(256), 0, s, frags, nfrag, L, half, k0, v0);
+    size_t tmp = 0;
+    VCT_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, k0, k1, v0, v1, (int)nfrag, 0, (int)(3u * L), s));
+    VCT_TRY(ensure(c->sort_tmp, tmp));
+    VCT_HIP(hipcub::DeviceRadixSort::SortPairs(c->sort_tmp.ptr, tmp, k0, k1, v0, v1, (int)nfrag, 0, (int)(3u * L), s));
+    hipLaunchKernelGGL(k_svo_node_count<Key>, dim3(nblocks), dim3(256), 0, s, (const Key*)k1, nfrag, L,
+                       (unsigned long long*)c->counts.ptr);
+    hipLaunchKernelGGL(k_svo_node_scan, dim3(L), dim3(1024), 0, s, (unsigned long long*)c->counts.ptr, nblocks,
+                       (unsigned long long*)c->totals.ptr);
+    VCT_HIP(hipGetLastError());
+    return VCT_OK;
+}
+
+template <typename Key>
+static void svo_nodes(vct_ctx* c, hipStream_t s, uint32_t nfrag, uint32_t L, uint2* pool)
+{
+    hipLaunchKernelGGL(k_svo_nodes<Key>, dim3(blocks_for(nfrag, kNodeKeys)), dim3(256), 0, s,
+                       (const Key*)c->rec_key[1].ptr, (const uint32_t*)c->rec_idx[1].ptr, nfrag, L,
+                       (const unsigned long long*)c->counts.ptr, (const unsigned long long*)c->totals.ptr, pool);
 }
 
 }  // namespace vct
@@ -622,77 +704,35 @@ vct_status vct_svo_build(vct_ctx* c, vct_stream stream)
     c->svo.pool_nodes = (uint32_t)cap;
     uint2* pool = (uint2*)c->svo.pool.ptr;
     const uint2* frags = (const uint2*)c->svo.frags.ptr;
-    uint32_t begin = 0, num = 8, counter = 0;
-    std::vector<uint32_t> level_begin, level_num;
-    VCT_TRY(ensure(c->counts, 8u * ((cap >> 6) + 8)));
-    VCT_TRY(ensure(c->offsets, 8u * ((cap >> 6) + 8)));
-    VCT_TRY(ensure(c->rec_idx[1], 4u * (size_t)(nfrag ? nfrag : 1)));
-    uint32_t* node_of = (uint32_t*)c->rec_idx[1].ptr;  // each fragment's node between flag passes
-    VCT_TRY(ensure(c->svo.counters, 16));
-    uint32_t* dev_counter = (uint32_t*)c->svo.counters.ptr;
-    VCT_HIP(hipMemsetAsync(dev_counter, 0, 4, s));
-    if (!c->pinned_word) VCT_HIP(hipHostMalloc(&c->pinned_word, kPinnedWordBytes, hipHostMallocDefault));
-    volatile uint32_t* host_counter = (volatile uint32_t*)c->pinned_word;
-    for (uint32_t i = 1; i <= L; ++i) {
-        if (num == 0) break;  // no node was flagged: the tree ends here (the reference's zero-group dispatches)
-        if ((uint64_t)begin + num > cap) return fail(VCT_ERR_CAPACITY, "octree node pool overflow (%llu nodes)", (unsigned long long)cap);
-        level_begin.push_back(begin);
-        level_num.push_back(num);
-        // octreeNodeInit.comp
-        hipLaunchKernelGGL(k_fill_u2, dim3(blocks_for(num)), dim3(256), 0, s, pool + begin, num, make_uint2(0u, 0u));
-        // octreeNodeFlag.comp
-        if (nfrag)
-            hipLaunchKernelGGL(k_svo_flag, dim3(blocks_for(nfrag)), dim3(256), 0, s, pool, frags, nfrag, L, i - 1u, half,
-                               node_of);
-        if (i == L) break;
-        // octreeNodeAlloc.comp + octreeNodeModifyArg.comp
-        const uint32_t waves = (num + 63) / 64;
-        uint32_t* wave_counts = (uint32_t*)c->counts.ptr;
-        uint32_t* wave_offsets = (uint32_t*)c->offsets.ptr;
-        hipLaunchKernelGGL(k_svo_alloc_count, dim3(blocks_for(num)), dim3(256), 0, s, pool, begin, num, wave_counts);
-        size_t tmp = 0;
-        VCT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, wave_counts, wave_offsets, (int)waves, s));
-        VCT_TRY(ensure(c->scan_tmp, tmp));
-        VCT_HIP(hipcub::DeviceScan::ExclusiveSum(c->scan_tmp.ptr, tmp, wave_counts, wave_offsets, (int)waves, s));
-        hipLaunchKernelGGL(k_svo_alloc_assign, dim3(blocks_for(num)), dim3(256), 0, s, pool, begin, num, wave_offsets,
-                           counter);
-        hipLaunchKernelGGL(k_svo_advance, dim3(1), dim3(1), 0, s, wave_offsets, wave_counts, waves, dev_counter);
-        VCT_HIP(hipMemcpyAsync((void*)host_counter, dev_counter, 4, hipMemcpyDeviceToHost, s));
+    // sizes per depth, then the pool
+    unsigned long long reached[kSvoMaxDepth] = {};  // nodes that some fragment reaches
+    if (nfrag) {
+        if (L <= 10) VCT_TRY(svo_sort<uint32_t>(c, s, frags, nfrag, L, half));
+        else VCT_TRY(svo_sort<unsigned long long>(c, s, frags, nfrag, L, half));
+        if (!c->pinned_word) VCT_HIP(hipHostMalloc(&c->pinned_word, kPinnedWordBytes, hipHostMallocDefault));
+        VCT_HIP(hipMemcpyAsync(c->pinned_word, c->totals.ptr, 8u * L, hipMemcpyDeviceToHost, s));
         VCT_HIP(hipStreamSynchronize(s));
-        counter = *host_counter;
-        begin += num;
-        num = (counter << 3) + 8u - begin;
+        for (uint32_t e = 0; e < L; ++e) reached[e] = ((volatile unsigned long long*)c->pinned_word)[e];
+    }
+    // depth e's nodes: the eight of the root, then eight per node reached above
+    std::vector<uint32_t> level_begin, level_num;
+    uint64_t total = 0;
+    for (uint32_t e = 0; e < L; ++e) {
+        const uint64_t num = e ? 8ull * reached[e - 1] : 8ull;
+        if (num == 0) break;  // no fragment: the tree ends here (the reference's zero-group dispatches)
+        if (total + num > cap) return fail(VCT_ERR_CAPACITY, "octree node pool overflow (%llu nodes)", (unsigned long long)cap);
+        level_begin.push_back((uint32_t)total);
+        level_num.push_back((uint32_t)num);
+        total += num;
+    }
+    // octreeNodeInit.comp
+    hipLaunchKernelGGL(k_fill_u2, dim3(blocks_for(total)), dim3(256), 0, s, pool, (uint32_t)total, make_uint2(0u, 0u));
+    if (nfrag) {
+        if (L <= 10) svo_nodes<uint32_t>(c, s, nfrag, L, pool);
+        else svo_nodes<unsigned long long>(c, s, nfrag, L, pool);
     }
     VCT_HIP(hipGetLastError());
-    const uint64_t total = ((uint64_t)counter << 3) + 8u;
-    if (total > cap) return fail(VCT_ERR_CAPACITY, "octree node pool overflow");
     c->svo.node_count = (uint32_t)total;
-    // octreeNodeLeafWrite.comp (fragment-ordered running average)
-    if (nfrag) {
-        for (int b = 0; b < 2; ++b) {
-            VCT_TRY(ensure(c->rec_key[b], 8u * (size_t)nfrag));
-        }
-        // key bits: fragment index below, leaf index above; a leaf index is
-        // below total - 1, so the all-ones `none` is above every real key
-        auto bits = [](unsigned long long v) {
-            int b = 0;
-            while (b < 64 && (v >> b) != 0ull) ++b;
-            return b;
-        };
-        const uint32_t fbits = (uint32_t)std::max(1, bits(nfrag - 1u));
-        const int end_bit = (int)fbits + bits(total);
-        const unsigned long long none = end_bit >= 64 ? ~0ull : (1ull << end_bit) - 1ull;
-        unsigned long long* k0 = (unsigned long long*)c->rec_key[0].ptr;
-        unsigned long long* k1 = (unsigned long long*)c->rec_key[1].ptr;
-        hipLaunchKernelGGL(k_svo_leaf_keys, dim3(blocks_for(nfrag)), dim3(256), 0, s, pool, frags, nfrag, R, half,
-                           fbits, none, k0);
-        size_t tmp = 0;
-        VCT_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, tmp, k0, k1, (int)nfrag, 0, end_bit, s));
-        VCT_TRY(ensure(c->sort_tmp, tmp));
-        VCT_HIP(hipcub::DeviceRadixSort::SortKeys(c->sort_tmp.ptr, tmp, k0, k1, (int)nfrag, 0, end_bit, s));
-        hipLaunchKernelGGL(k_svo_leaf_apply, dim3(blocks_for(nfrag)), dim3(256), 0, s, pool, frags, k1, nfrag, fbits,
-                           none);
-    }
     // octreeNodeMipmapWrite.comp for i = 2..L (OctreeBuilder.cpp:328-344). The
     // target of pass i is the node whose descent resolution equals i (quirk:
     // only i in {2, 4, 8} exist) or 2^(i-1); that node sits at depth
