@@ -363,7 +363,7 @@ __global__ __launch_bounds__(kExpandBlock) void k_phase_count(const SceneDev* __
         for (int k = 0; k < 9; ++k) p[k] = S.soup_pos[9u * t + k] - S.grid_min[k % 3];
         const int lo[3] = {0, 0, 0}, hi[3] = {S.res - 1, S.res - 1, S.res - 1};
         TriSetup st;
-        if (tri_setup(p, S.vs, lo, hi, st)) n = (unsigned long long)st.nu * st.nv * (unsigned long long)S.samples;
+        if (tri_setup(p, S.vs, S.samples, lo, hi, st)) n = (unsigned long long)st.nu * st.nv * (unsigned long long)S.samples;
     }
     const unsigned long long below = expand_block(n, &block_sums[blockIdx.x]);
     in_block[blockIdx.x * kExpandBlock + threadIdx.x] = below;
@@ -379,7 +379,8 @@ __global__ __launch_bounds__(1024) void k_phase_total(unsigned long long* __rest
 // Every covered sample of the batch proposes its (scene-local) triangle for
 // its voxel; the smallest index wins (k_dense_raster per scene). 16 scenes of
 // 5k to 60k triangles: 364 us with a search per lane between the block's first
-// and last triangles, 360 us so; the scan's two launches are gone.
+// and last triangles, 360 us so (the scan's two launches are gone), 252 us
+// since tri_setup's range keeps to the samples near the triangle.
 __global__ __launch_bounds__(256) void k_phase_raster_flat(const SceneDev* __restrict__ scenes,
                                                            const uint32_t* __restrict__ tri_start, uint32_t nscenes,
                                                            uint32_t ntris, Expansion E,
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(256) void k_phase_raster_flat(const SceneDev* __res
         for (int k = 0; k < 9; ++k) p[k] = S.soup_pos[9u * t + k] - S.grid_min[k % 3];
         const int rlo[3] = {0, 0, 0}, rhi[3] = {S.res - 1, S.res - 1, S.res - 1};
         TriSetup st;
-        if (!tri_setup(p, S.vs, rlo, rhi, st)) continue;
+        if (!tri_setup(p, S.vs, S.samples, rlo, rhi, st)) continue;
         float fp[3];
         double lam[3];
         if (!tri_sample(p, st, S.vs, S.samples, (uint32_t)(wi - E(g)), fp, lam)) continue;

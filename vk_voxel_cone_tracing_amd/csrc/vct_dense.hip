@@ -65,7 +65,8 @@ __global__ __launch_bounds__(kExpandBlock) void k_dense_count(const float* __res
             tpos[9u * t + k] = p[k];
         }
         TriSetup s;
-        if (tri_setup(p, R.vs, R.lo, R.hi, s)) n = (unsigned long long)s.nu * s.nv * (unsigned long long)R.samples;
+        if (tri_setup(p, R.vs, R.samples, R.lo, R.hi, s))
+            n = (unsigned long long)s.nu * s.nv * (unsigned long long)R.samples;
     }
     const unsigned long long below = expand_block(n, &block_sums[blockIdx.x]);
     in_block[blockIdx.x * kExpandBlock + threadIdx.x] = below;
@@ -102,7 +103,7 @@ __global__ __launch_bounds__(256) void k_dense_raster(const float* __restrict__ 
         float p[9];
         for (int k = 0; k < 9; ++k) p[k] = tpos[9u * t + k];
         TriSetup s;
-        if (!tri_setup(p, R.vs, R.lo, R.hi, s)) continue;
+        if (!tri_setup(p, R.vs, R.samples, R.lo, R.hi, s)) continue;
         float fp[3];
         double lam[3];
         if (!tri_sample(p, s, R.vs, R.samples, (uint32_t)(wi - E(t)), fp, lam)) continue;

@@ -91,7 +91,7 @@ __device__ __forceinline__ unsigned long long expand_scan(unsigned long long* su
 // last t with at(t) <= item. The whole wave must call it. The wave's first
 // triangle comes from a 64-way search (three dependent reads for 2^18
 // triangles, not eighteen: the opacity raster of a 128^3 x 6 level frame 44 ->
-// 37 us); the lanes then search the next 64 starts, held one
+// 37 us, tri_setup's general range taken); the lanes then search the next 64 starts, held one
 // per lane, and only lanes past those search memory by themselves (where most
 // triangles have no items).
 template <typename At>

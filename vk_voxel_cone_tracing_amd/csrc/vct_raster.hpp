@@ -52,8 +52,27 @@ __device__ __forceinline__ bool edge_covered(double w, double du, double dv)
 }
 
 // Triangle setup against the inclusive cell box [lo, hi]. Returns false for
-// degenerate triangles or an empty cell range.
-__device__ __forceinline__ bool tri_setup(const float* p, float vs, const int lo[3], const int hi[3], TriSetup& s)
+// degenerate triangles or a cell range that holds no covered sample.
+//
+// The cell range only has to hold every cell with a covered sample: the order
+// of the covered ones does not depend on the others. The general range is the
+// bounding box's cells and one more on each side. Where the rounding of the
+// edge functions can be bounded it is the cells with a sample within 1/16
+// voxel of the bounding box, a quarter or less of the items for triangles of a
+// voxel or two: cover pass of 1M triangles at 2^9 per axis 622 -> 235 us; dense
+// raster of 300k at 256^3 132 -> 44 us; opacity raster of six 128^3 levels 37
+// -> 22 us, injection 115 -> 68 us.
+//  * A sample 1/32 voxel or more outside the box (the rest is for rounding
+//    here: the reciprocal, product and sample position err by less than 2^-5.6
+//    voxel up to 2^16 voxels from the origin) is not covered: of the two edges
+//    at the vertex nearest it along the axis, whose angle has a sine of at
+//    least area / (2 E^2) for extent E, one is at least 2^-5 area / (4 E^2)
+//    voxel from the sample on its outer side, and the edge function's sign is
+//    right at distances above 2^-51 times the sample's from the vertex, which
+//    is below 2^18 voxels.
+//  * area > 2^-20 E^2 keeps 2^-27 apart from 2^-33.
+__device__ __forceinline__ bool tri_setup(const float* p, float vs, int samples, const int lo[3], const int hi[3],
+                                          TriSetup& s)
 {
 #pragma clang fp contract(off)
     s.axis = dominant_axis(p);
@@ -81,19 +100,32 @@ __device__ __forceinline__ bool tri_setup(const float* p, float vs, const int lo
     const float umax = fmaxf(p[s.u], fmaxf(p[3 + s.u], p[6 + s.u]));
     const float vmin = fminf(p[s.v], fminf(p[3 + s.v], p[6 + s.v]));
     const float vmax = fmaxf(p[s.v], fmaxf(p[3 + s.v], p[6 + s.v]));
-    // clamp before the integer conversion so that far-away geometry cannot overflow
-    const float lim = 1.0e9f;
-    long cu_lo = (long)floorf(fmaxf(umin / vs, -lim)) - 1, cu_hi = (long)floorf(fminf(umax / vs, lim)) + 1;
-    long cv_lo = (long)floorf(fmaxf(vmin / vs, -lim)) - 1, cv_hi = (long)floorf(fminf(vmax / vs, lim)) + 1;
-    if (cu_lo < lo[s.u]) cu_lo = lo[s.u];
-    if (cu_hi > hi[s.u]) cu_hi = hi[s.u];
-    if (cv_lo < lo[s.v]) cv_lo = lo[s.v];
-    if (cv_hi > hi[s.v]) cv_hi = hi[s.v];
+    const float inv = 1.0f / vs, far = 65536.0f;
+    const float ua = umin * inv, ub = umax * inv, va = vmin * inv, vb = vmax * inv;
+    const double extent = fmax((double)umax - umin, (double)vmax - vmin);
+    int cu_lo, cu_hi, cv_lo, cv_hi;
+    if (fabsf(ua) <= far && fabsf(ub) <= far && fabsf(va) <= far && fabsf(vb) <= far &&
+        area > extent * extent * 0x1p-20) {
+        // the samples' offsets in their cell, widened by 1/16
+        const float first = samples == 4 ? 0.125f - 0.0625f : 0.5f - 0.0625f;
+        const float last = samples == 4 ? 0.875f + 0.0625f : 0.5f + 0.0625f;
+        cu_lo = max((int)ceilf(ua - last), lo[s.u]);
+        cu_hi = min((int)floorf(ub - first), hi[s.u]);
+        cv_lo = max((int)ceilf(va - last), lo[s.v]);
+        cv_hi = min((int)floorf(vb - first), hi[s.v]);
+    } else {
+        // clamp before the integer conversion so that far-away geometry cannot overflow
+        const float lim = 1.0e9f;
+        cu_lo = max((int)floorf(fminf(fmaxf(umin / vs, -lim), lim)) - 1, lo[s.u]);
+        cu_hi = min((int)floorf(fmaxf(fminf(umax / vs, lim), -lim)) + 1, hi[s.u]);
+        cv_lo = max((int)floorf(fminf(fmaxf(vmin / vs, -lim), lim)) - 1, lo[s.v]);
+        cv_hi = min((int)floorf(fmaxf(fminf(vmax / vs, lim), -lim)) + 1, hi[s.v]);
+    }
     if (cu_hi < cu_lo || cv_hi < cv_lo) return false;
-    s.cu_lo = (int)cu_lo;
-    s.cv_lo = (int)cv_lo;
-    s.nu = (int)(cu_hi - cu_lo + 1);
-    s.nv = (int)(cv_hi - cv_lo + 1);
+    s.cu_lo = cu_lo;
+    s.cv_lo = cv_lo;
+    s.nu = cu_hi - cu_lo + 1;
+    s.nv = cv_hi - cv_lo + 1;
     return true;
 }
 

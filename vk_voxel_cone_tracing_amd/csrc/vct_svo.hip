@@ -56,7 +56,7 @@ __global__ void k_svo_count(const float* __restrict__ npos, uint32_t ntris, SvoR
     for (int k = 0; k < 9; ++k) p[k] = npos[9u * t + k];
     TriSetup s;
     unsigned long long n = 0;
-    if (tri_setup(p, R.vs, R.lo, R.hi, s)) n = (unsigned long long)s.nu * s.nv * (unsigned long long)R.samples;
+    if (tri_setup(p, R.vs, R.samples, R.lo, R.hi, s)) n = (unsigned long long)s.nu * s.nv * (unsigned long long)R.samples;
     counts[t] = n;
 }
 
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_svo_cover(const float* __restrict__ npo
     for (int k = 0; k < 9; ++k) p[k] = npos[9u * t + k];
     TriSetup s;
     uint32_t c = 0;
-    if (tri_setup(p, R.vs, R.lo, R.hi, s)) {
+    if (tri_setup(p, R.vs, R.samples, R.lo, R.hi, s)) {
         float fp[3];
         double lam[3];
         c = tri_sample(p, s, R.vs, R.samples, (uint32_t)(wi - offsets[t]), fp, lam) ? 1u : 0u;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void k_svo_write(const float* __restrict__ npo
     float p[9];
     for (int k = 0; k < 9; ++k) p[k] = npos[9u * t + k];
     TriSetup s;
-    if (!tri_setup(p, R.vs, R.lo, R.hi, s)) return;
+    if (!tri_setup(p, R.vs, R.samples, R.lo, R.hi, s)) return;
     float fp[3];
     double lam[3];
     if (!tri_sample(p, s, R.vs, R.samples, (uint32_t)(wi - offsets[t]), fp, lam)) return;

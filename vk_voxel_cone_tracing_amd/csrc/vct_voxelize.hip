@@ -117,7 +117,7 @@ __global__ __launch_bounds__(kExpandBlock) void k_count(const float* __restrict_
 #pragma unroll
         for (int k = 0; k < 9; ++k) p[k] = pos[9u * t + k];
         TriSetup s;
-        if (tri_setup(p, P.voxel_size, P.lo, P.hi, s))
+        if (tri_setup(p, P.voxel_size, P.samples, P.lo, P.hi, s))
             n = (unsigned long long)s.nu * s.nv * (unsigned long long)P.samples;
     }
     const uint32_t b = slot * gridDim.x + blockIdx.x;
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void k_raster_opacity(const float* __restrict_
 #pragma unroll
         for (int k = 0; k < 9; ++k) p[k] = pos[9u * t + k];
         TriSetup s;
-        if (!tri_setup(p, P.voxel_size, P.lo, P.hi, s)) continue;
+        if (!tri_setup(p, P.voxel_size, P.samples, P.lo, P.hi, s)) continue;
         float fp[3];
         double lam[3];
         if (!tri_sample(p, s, P.voxel_size, P.samples, it.sample, fp, lam)) continue;
@@ -264,7 +264,8 @@ __global__ __launch_bounds__(256) void k_raster_inject(const float* __restrict__
     // The records' places in the buffer come from one atomic per workgroup and
     // trip: the counter is one address, which takes some 90 million atomics a
     // second, and one per wave was the kernel's bound (128^3 x 6 levels, 21 260
-    // triangles: 189 -> 115 us).
+    // triangles: 189 -> 115 us; 68 us
+    // since tri_setup's range keeps to the samples near the triangle).
     for (unsigned long long base = (unsigned long long)blockIdx.x * 256u; base < n; base += stride) {
         const unsigned long long wi = base + threadIdx.x;
         Record out[6];
@@ -284,7 +285,7 @@ __global__ __launch_bounds__(256) void k_raster_inject(const float* __restrict__
 #pragma unroll
             for (int k = 0; k < 9; ++k) p[k] = pos[9u * t + k];
             TriSetup s;
-            if (!tri_setup(p, P.voxel_size, P.lo, P.hi, s)) return;
+            if (!tri_setup(p, P.voxel_size, P.samples, P.lo, P.hi, s)) return;
             float fp[3];
             double lam[3];
             if (!tri_sample(p, s, P.voxel_size, P.samples, it.sample, fp, lam)) return;
