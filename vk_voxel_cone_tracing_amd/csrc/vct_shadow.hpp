@@ -22,39 +22,38 @@ struct LightParams {
     int width, height;
 };
 
-__device__ __forceinline__ float fetch_depth(const LightParams& L, int i, int j)
-{
-    if (i < 0 || j < 0 || i >= L.width || j >= L.height) return 0.0f;  // CLAMP_TO_BORDER, opaque black
-    return L.depth[(size_t)j * (size_t)L.width + (size_t)i];
-}
-
-__device__ __forceinline__ float shadow_tap(const LightParams& L, float s, float t, bool compare, float ref)
+// A tap's first texel and weight along one axis.
+__device__ __forceinline__ void tap_origin(float at, float size, int& first, float& frac)
 {
 #pragma clang fp contract(off)
-    float uu = s * (float)L.width - 0.5f;
-    float vv = t * (float)L.height - 0.5f;
-    float fu = floorf(uu), fv = floorf(vv);
-    float a = uu - fu, b = vv - fv;
-    fu = fminf(fmaxf(fu, -4.0f), (float)L.width + 4.0f);
-    fv = fminf(fmaxf(fv, -4.0f), (float)L.height + 4.0f);
-    int i0 = (int)fu, j0 = (int)fv;
-    float t00 = fetch_depth(L, i0, j0), t10 = fetch_depth(L, i0 + 1, j0);
-    float t01 = fetch_depth(L, i0, j0 + 1), t11 = fetch_depth(L, i0 + 1, j0 + 1);
-    if (compare) {
-        bool in00 = i0 >= 0 && j0 >= 0 && i0 < L.width && j0 < L.height;
-        bool in10 = i0 + 1 >= 0 && j0 >= 0 && i0 + 1 < L.width && j0 < L.height;
-        bool in01 = i0 >= 0 && j0 + 1 >= 0 && i0 < L.width && j0 + 1 < L.height;
-        bool in11 = i0 + 1 >= 0 && j0 + 1 >= 0 && i0 + 1 < L.width && j0 + 1 < L.height;
-        t00 = (!in00 || ref <= t00) ? 1.0f : 0.0f;
-        t10 = (!in10 || ref <= t10) ? 1.0f : 0.0f;
-        t01 = (!in01 || ref <= t01) ? 1.0f : 0.0f;
-        t11 = (!in11 || ref <= t11) ? 1.0f : 0.0f;
-    }
+    const float u = at * size - 0.5f, f = floorf(u);
+    frac = u - f;
+    first = (int)fminf(fmaxf(f, -4.0f), size + 4.0f);
+}
+
+// A texel as a tap weighs it: its depth, or how it compares.
+__device__ __forceinline__ float tap_texel(const LightParams& L, int i, int j, bool compare, float ref)
+{
+    const bool in = i >= 0 && j >= 0 && i < L.width && j < L.height;  // CLAMP_TO_BORDER, opaque black
+    const float t = in ? L.depth[(size_t)j * (size_t)L.width + (size_t)i] : 0.0f;
+    return compare ? ((!in || ref <= t) ? 1.0f : 0.0f) : t;
+}
+
+__device__ __forceinline__ float tap_weigh(float a, float b, float t00, float t10, float t01, float t11)
+{
+#pragma clang fp contract(off)
     float r = ((1.0f - a) * (1.0f - b)) * t00;
     r = r + (a * (1.0f - b)) * t10;
     r = r + ((1.0f - a) * b) * t01;
     r = r + (a * b) * t11;
     return r;
+}
+
+// Five texels of one row of the window.
+__device__ __forceinline__ void window_row(const LightParams& L, int i0, int j, bool compare, float ref, float row[5])
+{
+#pragma unroll
+    for (int k = 0; k < 5; ++k) row[k] = tap_texel(L, i0 + k, j, compare, ref);
 }
 
 // shadow.glsl:28-36 calcVisibility + PCF16 (:14-26)
@@ -79,18 +78,49 @@ __device__ __forceinline__ float visibility(const LightParams& L, const float po
     const float sx = 1.0f / (float)L.width;
     const float sy = 1.0f / (float)L.height;
     // offsets -1.5, -0.5, 0.5, 1.5 (exact in float), y outer as in the
-    // reference; integer counters let the 16 taps unroll so their fetches
-    // are in flight together
-    float sum = 0.0f;
+    // reference. The taps' columns depend on x alone and their rows on y alone,
+    // and as a rule the four columns (rows) are consecutive: then all taps read
+    // one window of 5 x 5 texels, each fetched and compared once (64 fetches
+    // tap by tap). Where rounding or the border's clamp makes them other than
+    // consecutive, the taps fetch for themselves. Bound by the fetches and
+    // their bounds tests: octree fragments of 1M triangles at 2^9, shadow map
+    // 2048^2, 694 -> 304 us; injection at 128^3 x 6 levels 68 -> 54 us.
+    float fx[4], fy[4];
+    int x0[4], y0[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float y = -1.5f + (float)j;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float x = -1.5f + (float)i;
-            sum = sum + shadow_tap(L, xy[0] + x * sx, xy[1] + y * sy, compare, ref);
-        }
+    for (int k = 0; k < 4; ++k) {
+        const float off = -1.5f + (float)k;
+        tap_origin(xy[0] + off * sx, (float)L.width, x0[k], fx[k]);
+        tap_origin(xy[1] + off * sy, (float)L.height, y0[k], fy[k]);
     }
+    bool window = true;
+#pragma unroll
+    for (int k = 1; k < 4; ++k) window = window && x0[k] == x0[0] + k && y0[k] == y0[0] + k;
+    if (window) {
+        float sum = 0.0f, row[2][5];
+        window_row(L, x0[0], y0[0], compare, ref, row[0]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            window_row(L, x0[0], y0[0] + j + 1, compare, ref, row[(j + 1) & 1]);
+            const float* r0 = row[j & 1];
+            const float* r1 = row[(j + 1) & 1];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum = sum + tap_weigh(fx[i], fy[j], r0[i], r0[i + 1], r1[i], r1[i + 1]);
+        }
+        return sum * 0.0625f;
+    }
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int j = 0; j < 4; ++j)
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i) {
+            int i0, j0;
+            float a, b;
+            tap_origin(xy[0] + (-1.5f + (float)i) * sx, (float)L.width, i0, a);
+            tap_origin(xy[1] + (-1.5f + (float)j) * sy, (float)L.height, j0, b);
+            sum = sum + tap_weigh(a, b, tap_texel(L, i0, j0, compare, ref), tap_texel(L, i0 + 1, j0, compare, ref),
+                                  tap_texel(L, i0, j0 + 1, compare, ref), tap_texel(L, i0 + 1, j0 + 1, compare, ref));
+        }
     return sum * 0.0625f;
 }
 
