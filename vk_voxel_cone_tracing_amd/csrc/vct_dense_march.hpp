@@ -353,27 +353,16 @@ __device__ __forceinline__ void pixel_setup(const Pyramid& P, const March& M, in
     albedo[2] = u8_to_f((diffuse >> 16) & 0xffu);
 }
 
-// A lane's part of the adjoint tape: cone i's samples from col + i * stride
-// (float4 units, one column of 64), its accumulated step count at
-// counts[i * 64] (kTapeOverflow when the march took more than cap steps).
-struct LaneTape {
-    float4* col;
-    size_t stride;
-    uint8_t* counts;
-    uint32_t cap;
-};
-
+// A lane's step count on the tape when its march took more steps than fit.
 constexpr uint8_t kTapeOverflow = 255;
 
 // One pixel of the dense trace: 16 (or 32) cones weighted by cos, output
-// (indirect diffuse x albedo x intensity, ambient occlusion). With a tape,
-// the counts of the cones it marches are written (the caller zeroes them).
+// (indirect diffuse x albedo x intensity, ambient occlusion).
 template <bool kF32, bool kAhead>
 __device__ __forceinline__ float4 dense_pixel(const void* __restrict__ data, const Pyramid& P, const March& M, int px,
                                               int py, int width, int height, const uint32_t* __restrict__ g_diffuse,
                                               const uint16_t* __restrict__ g_normal,
-                                              const float* __restrict__ g_depth, uint32_t& steps,
-                                              const LaneTape* lt = nullptr)
+                                              const float* __restrict__ g_depth, uint32_t& steps)
 {
     const size_t idx = (size_t)py * (size_t)width + (size_t)px;
     const float depth = g_depth[idx];
@@ -385,14 +374,7 @@ __device__ __forceinline__ float4 dense_pixel(const void* __restrict__ data, con
         const float* d = cone_dir(M, i);
         const float ct = normal[0] * d[0] + normal[1] * d[1] + normal[2] * d[2];
         if (ct < 0.0f) continue;
-        f4 c;
-        if (lt) {
-            TapeSlot t{lt->col + (size_t)i * lt->stride, lt->cap, 0u};
-            c = march<kF32, kAhead>(data, P, M, start, d, steps, &t);
-            lt->counts[i * 64] = t.count > lt->cap ? kTapeOverflow : (uint8_t)t.count;
-        } else {
-            c = march<kF32, kAhead>(data, P, M, start, d, steps);
-        }
+        const f4 c = march<kF32, kAhead>(data, P, M, start, d, steps);
         ind.x += c.x * ct;
         ind.y += c.y * ct;
         ind.z += c.z * ct;

@@ -12,8 +12,8 @@
 // fragment emits one record per written face texel keyed by
 // (texel address in the volume, work index), a radix sort groups the records
 // by texel in fragment order (a texel belongs to one level, whose work items
-// keep their order), and one lane per texel applies the running average (RGBA8)
-// or the FP32 sum/count mean (RGBA16F) in that order.
+// keep their order), and one lane per texel (a wave for a long run) applies the
+// running average (RGBA8) or the FP32 sum/count mean (RGBA16F) in that order.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
