@@ -145,10 +145,11 @@ constexpr int tail_edge()
 }
 
 template <bool kF32>
-constexpr int tail_texels()  // the tail's levels, the last excepted
+constexpr int tail_texels()  // the tail's levels that another level is made from: all but the last, 1^3
 {
-    const int e = tail_edge<kF32>();
-    return e * e * e + e * e * e / 8 + e * e * e / 64 + 8;
+    int texels = 0;
+    for (int e = tail_edge<kF32>(); e > 1; e /= 2) texels += e * e * e;
+    return texels;
 }
 
 // Face f of levels m, m + 1, ..., nlevels - 1 (res >> m <= tail_edge), level l
@@ -178,7 +179,7 @@ __device__ __forceinline__ void dense_mip_tail(void* data, const unsigned long l
             }
             const f4 o = dense_mip_any_face(v, f);
             dense_store<kF32>(dst, dense_mip_index(n, x, y, z), o);
-            dense_store<kF32>(here, (size_t)i, o);
+            if (m + 1 < nlevels) dense_store<kF32>(here, (size_t)i, o);
         }
         __syncthreads();
         below = here;
@@ -186,9 +187,9 @@ __device__ __forceinline__ void dense_mip_tail(void* data, const unsigned long l
     }
 }
 
-// The arithmetic of one destination texel with one face at a time (the face loop is not
-// unrolled and each pair's children are loaded by computed index), for
-// kernels that must keep few registers live: the persistent batched launch,
+// The arithmetic of one destination texel with one face at a time (the face
+// loop is not unrolled and each pair's children are loaded by computed index),
+// for kernels that must keep few registers live: the persistent batched launch,
 // whose pixel tiles would otherwise inherit the unrolled version's registers.
 template <bool kF32>
 __device__ __forceinline__ void dense_mip_texel_lean(const void* src, void* dst, int n, int x, int y, int z,
