@@ -558,7 +558,7 @@ vct_status vct_dense_trace_tape(vct_dense* grid, vct_stream stream, const vct_gb
  * one image size in one call (host arrays of views G-buffers and cameras, and
  * of device pointers to each view's output and tape, each tape of at least
  * tape_bytes): the same images and tapes, the views sharing the launches (one
- * per 16 views). */
+ * per 16 views). No views: nothing is done, and the arrays may be null. */
 vct_status vct_dense_trace_views(vct_dense* grid, vct_stream stream, uint32_t views, const vct_gbuffer* gbuffers,
                                  const vct_camera_ubo* cameras, const vct_dense_trace_desc* desc, float* const* outs,
                                  void* const* tapes, size_t tape_bytes);

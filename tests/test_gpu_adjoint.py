@@ -349,3 +349,24 @@ def test_autograd_function_matches_c_abi_gradient():
         for g, r in ((ta.grad, ra), (to.grad, rop)):
             g = g.cpu().numpy().astype(np.float64)
             assert np.linalg.norm(g - r) / np.linalg.norm(r) < 1e-5, mode
+
+
+def test_no_views():
+    """An empty stack of views renders an empty image, with zero gradients."""
+    import torch
+    from vk_voxel_cone_tracing_amd import adjoint
+
+    ta = torch.rand((8, 8, 8, 3), device="cuda", requires_grad=True)
+    to = torch.rand((8, 8, 8), device="cuda", requires_grad=True)
+    empty = lambda dtype, *s: torch.empty((0, H, W) + s, dtype=dtype, device="cuda")  # noqa: E731
+    for mode in ("no grad", "tape", "keep", "recompute"):
+        ta.grad = to.grad = None
+        with torch.set_grad_enabled(mode != "no grad"):
+            out = adjoint.render(ta, to, empty(torch.int32), empty(torch.int16, 4), empty(torch.float32),
+                                 torch.empty((0, 36)), (0.0, 0.0, 0.0), 1.0, adjoint.TraceParams(*TD),
+                                 recompute=mode == "recompute", tape=mode != "keep")
+        assert out.shape == (0, H, W, 4)
+        if mode != "no grad":
+            out.sum().backward()
+            for t in (ta, to):
+                assert t.grad.shape == t.shape and not t.grad.any(), mode

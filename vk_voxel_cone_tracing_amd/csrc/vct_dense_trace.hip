@@ -151,8 +151,9 @@ static vct_status trace_views(vct_dense* g, hipStream_t s, uint32_t views, const
                               const vct_camera_ubo* cams, const vct_dense_trace_desc* d, float* const* outs,
                               void* const* tapes, size_t tape_bytes, unsigned long long* samples)
 {
-    if (!g || !gbs || !cams || !d || !outs) return fail(VCT_ERR_INVALID_ARGUMENT, "null argument");
-    if (!views) return VCT_OK;
+    if (!g || !d) return fail(VCT_ERR_INVALID_ARGUMENT, "null argument");
+    if (!views) return VCT_OK;  // the arrays of no views may be null (an empty vector's data())
+    if (!gbs || !cams || !outs) return fail(VCT_ERR_INVALID_ARGUMENT, "null argument");
     const uint32_t W = gbs[0].width, H = gbs[0].height;
     for (uint32_t v = 0; v < views; ++v) {
         if (!outs[v] || (tapes && !tapes[v])) return fail(VCT_ERR_INVALID_ARGUMENT, "null argument");
