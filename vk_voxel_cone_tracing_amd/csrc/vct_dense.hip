@@ -306,11 +306,20 @@ vct_status vct_dense_voxelize(vct_dense* g, vct_stream stream, const vct_mesh* m
     VCT_TRY(ensure(c->offsets, 8u * (size_t)nblocks));
     VCT_TRY(ensure(c->totals, 64));
     const size_t nv = (size_t)g->res * g->res * g->res;
-    const bool fresh = !g->winner.ptr;
     VCT_TRY(ensure(g->winner, 4u * nv));
-    if (fresh)  // every voxelization leaves the winners empty
+    // Every voxelization leaves the winners empty for the next; one that fails
+    // on the way leaves that to the next. A fill that is only recorded into a
+    // graph runs with the graph, so the calls after it fill again.
+    const bool fill = !g->winners_empty;
+    bool recorded = false;
+    g->winners_empty = false;
+    if (fill) {
+        hipStreamCaptureStatus capture;
+        VCT_HIP(hipStreamIsCapturing(s, &capture));
+        recorded = capture != hipStreamCaptureStatusNone;
         hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, s, (uint32_t*)g->winner.ptr,
                            nv, 0xffffffffu);
+    }
     const Expansion E{(const unsigned long long*)c->counts.ptr, (const unsigned long long*)c->offsets.ptr};
     auto* total = (unsigned long long*)c->totals.ptr;
     hipLaunchKernelGGL(k_dense_count, dim3(nblocks), dim3(kExpandBlock), 0, s, soup.pos, soup.count,
@@ -329,6 +338,7 @@ vct_status vct_dense_voxelize(vct_dense* g, vct_stream stream, const vct_mesh* m
     if (g->texel_bytes == 16) g->res >= 4 ? resolve(k_dense_resolve<true, 4>, 4) : resolve(k_dense_resolve<true, 1>, 1);
     else g->res >= 4 ? resolve(k_dense_resolve<false, 4>, 4) : resolve(k_dense_resolve<false, 1>, 1);
     VCT_HIP(hipGetLastError());
+    g->winners_empty = !recorded;
     return VCT_OK;
 }
 

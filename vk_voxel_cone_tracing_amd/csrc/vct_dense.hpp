@@ -13,6 +13,7 @@ struct vct_dense {
     size_t texels = 0;
     vct::DeviceBuffer data;
     vct::DeviceBuffer winner;
+    bool winners_empty = false;  // every voxel's winner is empty once the work launched so far has run
     vct::DeviceBuffer bwd_rec, bwd_hdr, bwd_start, bwd_ctr;  // the trace adjoint's sweep records
     vct_ctx* scratch = nullptr;  // vertex stage / raster scratch (no clipmap volumes)
 };
