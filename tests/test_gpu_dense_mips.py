@@ -1,7 +1,8 @@
 """The dense mip pyramid of random level-0 texels against a NumPy float32
 restatement, bit for bit, at every resolution where the launches change: the
-whole pyramid in the one-workgroup tail (2 to 32), one or two levels above it,
-and rows of 64 texels; RGBA8 and RGBA32F, and the batched launch's bricks."""
+whole pyramid in the one-workgroup tail (2 to 32, RGBA32F to 16), one or more
+levels above it, and rows of 64 texels; RGBA8 and RGBA32F, and the batched
+launch's bricks."""
 import ctypes as C
 
 import numpy as np

@@ -377,10 +377,10 @@ __global__ __launch_bounds__(1024) void k_phase_total(unsigned long long* __rest
 }
 
 // Every covered sample of the batch proposes its (scene-local) triangle for
-// its voxel; the smallest index wins (k_dense_raster per scene). 16 scenes of
-// 5k to 60k triangles: 364 us with a search per lane between the block's first
-// and last triangles, 360 us so (the scan's two launches are gone), 252 us
-// since tri_setup's range keeps to the samples near the triangle.
+// its voxel; the smallest index wins (k_dense_raster per scene). Bound by the
+// edge functions and the atomics. 16 scenes of 5k to 60k triangles: 252 us (a
+// search per lane between the block's first and last triangles was no slower
+// than the wave's, but took the scan's two launches).
 __global__ __launch_bounds__(256) void k_phase_raster_flat(const SceneDev* __restrict__ scenes,
                                                            const uint32_t* __restrict__ tri_start, uint32_t nscenes,
                                                            uint32_t ntris, Expansion E,

@@ -93,11 +93,12 @@ struct BlurStencil {
     float slope;
 };
 
-// Bound by HBM: two images read, one written. One lane per pixel, 64 x 4
-// pixels per workgroup, so a wave reads and writes whole 1 KB row pieces; the
-// 3x3 neighbours come from the L1. 1920x1080: 943 us (with tonemap) with the
-// 256 taps evaluated one by one, about 1000 texel loads a pixel; now 17 us, 34
-// with the tonemap's powers (100 MB, 5.9 and 2.9 TB/s).
+// Bound by HBM (two images read, one written), with the tonemap by its three
+// powers a pixel. One lane per pixel, 64 x 4 pixels per workgroup, so a wave
+// reads and writes whole 1 KB row pieces; the 3x3 neighbours come from the L1.
+// 1920x1080: 943 us (with tonemap) with the 256 taps evaluated one by one, about
+// 1000 texel loads a pixel; now 17 us, 34 with the tonemap's powers (100 MB, 5.9
+// and 2.9 TB/s).
 __global__ __launch_bounds__(256) void k_specular_blur(const float4* __restrict__ diffuse,
                                                        const float4* __restrict__ specular, int W, int H,
                                                        BlurStencil S, Tonemap T, float4* __restrict__ out)

@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) void k_svo_keys(const uint2* __restrict__ frag
     uint32_t p[3];
     frag_pos(v, half, p);
     const uint32_t top = (1u << L) - 1u;
-    auto spread = [](uint32_t c) -> Key {  // bit b to bit 3b
+    auto spread = [](uint32_t c) -> Key {  // bit b to bit 3b (the Morton code's steps)
         uint32_t r = c & 1023u;
         r = (r | (r << 16)) & 0x030000ffu;
         r = (r | (r << 8)) & 0x0300f00fu;

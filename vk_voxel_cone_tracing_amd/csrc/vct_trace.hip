@@ -935,7 +935,8 @@ struct SvoTraceParams {
 };
 
 // x / d for the constant d of a launch, r = 1 / d correctly rounded: the
-// quotient estimate and one residual correction round as the division does.
+// quotient estimate and one residual correction round as the division does
+// (Markstein's theorem).
 __device__ __forceinline__ float div_const(float x, float d, float r)
 {
     const float q = x * r;

@@ -263,9 +263,8 @@ __global__ __launch_bounds__(256) void k_raster_inject(const float* __restrict__
     const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
     // The records' places in the buffer come from one atomic per workgroup and
     // trip: the counter is one address, which takes some 90 million atomics a
-    // second, and one per wave was the kernel's bound (128^3 x 6 levels, 21 260
-    // triangles: 189 -> 115 us; 54 us since
-    // tri_setup's range and the shadow window).
+    // second, and with one per wave it was the kernel's bound. 128^3 x 6 levels,
+    // 21 260 triangles: 54 us.
     for (unsigned long long base = (unsigned long long)blockIdx.x * 256u; base < n; base += stride) {
         const unsigned long long wi = base + threadIdx.x;
         Record out[6];
@@ -414,9 +413,9 @@ struct Applied {
             return;
         }
         // the three quotients by the new count (1 to 256) from its correctly
-        // rounded reciprocal and one residual correction each, which rounds
-        // as the division does and keeps it off the chain from record to
-        // record (the reciprocal depends on the count only)
+        // rounded reciprocal and one residual correction each (Markstein's
+        // theorem), which rounds as the division does and keeps it off the
+        // chain from record to record (the reciprocal depends on the count only)
         const float d = w + 1.0f, r = 1.0f / d;
         x = average(x * w + vx, d, r);
         y = average(y * w + vy, d, r);
