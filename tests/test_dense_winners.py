@@ -1,66 +1,14 @@
 """The winners of the dense voxelizer are kept empty from one call to the next:
 filled by the first call, by the call after one that failed, and by every call
-after a fill that was only recorded into a graph. A host program stands in for
-the HIP runtime (its symbols come before the library's), so that no kernel
-runs, any launch can be made to fail, and the launches of a call are listed."""
+after a fill that was only recorded into a graph. The library's host code runs
+against a stand-in for the HIP runtime, with one of its launches failing."""
 import subprocess
-from pathlib import Path
 
 import pytest
 
-ROOT = Path(__file__).resolve().parents[1]
+import hip_stand_in
 
 MAIN = r"""
-#include <dlfcn.h>
-#include <cstdio>
-#include <cstdlib>
-#include <cstring>
-#include <map>
-#include <string>
-#include "vct.h"
-
-// ---- the HIP runtime, on host memory
-struct dim3 { unsigned x, y, z; };
-static std::map<const void*, std::string> names;
-static std::string launched, failing;
-static int last_error = 0, capturing = 0;
-static dim3 grid_, block_;
-static size_t shared_;
-static void* stream_;
-extern "C" {
-void** __hipRegisterFatBinary(const void*) { static void* h; return &h; }
-void __hipUnregisterFatBinary(void**) {}
-void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, void*, void*, int*)
-{
-    names[f] = name;
-}
-void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
-int __hipPushCallConfiguration(dim3 g, dim3 b, size_t m, void* s) { grid_ = g; block_ = b; shared_ = m; stream_ = s; return 0; }
-int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* m, void** s) { *g = grid_; *b = block_; *m = shared_; *s = stream_; return 0; }
-int hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, void*)
-{
-    const std::string& n = names[f];
-    if (!failing.empty() && n.find(failing) != std::string::npos) return last_error = 1;
-    launched += n + ' ';
-    return 0;
-}
-int hipGetLastError() { const int e = last_error; last_error = 0; return e; }
-const char* hipGetErrorString(int) { return "error"; }
-int hipMalloc(void** p, size_t n) { return (*p = calloc(1, n)) ? 0 : 2; }
-int hipFree(void* p) { free(p); return 0; }
-int hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
-int hipHostFree(void* p) { return hipFree(p); }
-int hipMemset(void* p, int v, size_t n) { memset(p, v, n); return 0; }
-int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*) { memcpy(d, s, n); return 0; }
-int hipGetDevice(int* d) { *d = 0; return 0; }
-int hipDeviceSynchronize() { return 0; }
-int hipStreamSynchronize(void*) { return 0; }
-int hipGetSymbolAddress(void** p, const void*) { static char c; *p = &c; return 0; }
-int hipStreamIsCapturing(void*, int* s) { *s = capturing; return 0; }
-}
-
-#define CALL(name) ((decltype(&name))dlsym(lib, #name))
-
 int main(int, char** argv)
 {
     void* lib = dlopen(argv[1], RTLD_LAZY | RTLD_LOCAL);
@@ -91,7 +39,8 @@ int main(int, char** argv)
         const bool done = CALL(vct_dense_voxelize)(g, nullptr, &mesh) == VCT_OK;
         const bool filled = launched.find("k_fill_u32") != std::string::npos;
         if (done != ok || filled != fills) {
-            printf("%s: %s, winners %sfilled [%s]\n", what, done ? "done" : "failed", filled ? "" : "not ", launched.c_str());
+            printf("%s: %s, winners %sfilled [%s]\n", what, done ? "done" : "failed", filled ? "" : "not ",
+                   launched.c_str());
             exit(1);
         }
     };
@@ -126,16 +75,11 @@ int main(int, char** argv)
 
 @pytest.fixture(scope="module")
 def host(tmp_path_factory):
-    d = tmp_path_factory.mktemp("winners")
-    (d / "main.cpp").write_text(MAIN)
-    exe = str(d / "host")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-rdynamic", f"-I{ROOT / 'include'}", str(d / "main.cpp"), "-ldl",
-                    "-o", exe], check=True)
-    return exe
+    return hip_stand_in.build(tmp_path_factory.mktemp("winners"), MAIN)
 
 
-@pytest.mark.parametrize("failing", ["k_fill_u32", "k_dense_count", "k_dense_total", "k_dense_raster", "k_dense_resolve",
-                                     ""])
+@pytest.mark.parametrize("failing", ["k_fill_u32", "k_dense_count", "k_dense_total", "k_dense_raster",
+                                     "k_dense_resolve", ""])
 def test_winners_are_filled_after_a_failure(host, failing):
     from vk_voxel_cone_tracing_amd import _abi
 

@@ -590,6 +590,12 @@ __device__ __forceinline__ void pixel_in(const TraceParams& P, size_t idx, int p
     for (int k = 0; k < 3; ++k) I.start[k] = I.world[k] + I.normal[k] * vs * P.start_offset;
 }
 
+// The modes that march the diffuse cones.
+__host__ __device__ __forceinline__ bool wants_diffuse(const TraceParams& P)
+{
+    return P.mode == 4u || P.mode == 5u || P.mode == 7u || P.mode == 8u;
+}
+
 __device__ __forceinline__ bool wants_specular(const TraceParams& P, const PixelIn& I)
 {
     return (P.mode == 6u || P.mode == 8u) && (I.sc[0] > 1e-6f || I.sc[1] > 1e-6f || I.sc[2] > 1e-6f) &&
@@ -661,7 +667,7 @@ __global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void k_trace(
     const float depth = in_image ? g_depth[idx] : 1.0f;
     const bool surface = depth != 1.0f;
     const int ncones = P.cones32 ? 32 : 16;
-    const bool want_diffuse = (P.mode == 4u || P.mode == 5u || P.mode == 7u || P.mode == 8u);
+    const bool want_diffuse = wants_diffuse(P);
     const bool want_direct = (P.mode == 4u || P.mode == 5u || P.mode == 8u);
     uint32_t steps = 0;
     PixelIn I;
@@ -1082,7 +1088,7 @@ __global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void k_svo_trace(
     const float depth = in_image ? g_depth[idx] : 1.0f;
     const bool surface = depth != 1.0f;
     const int ncones = P.cones32 ? 32 : 16;
-    const bool want_diffuse = (P.mode == 4u || P.mode == 5u || P.mode == 7u || P.mode == 8u);
+    const bool want_diffuse = wants_diffuse(P);
     uint32_t steps = 0;
     PixelIn I;
     f4 ind = {0.0f, 0.0f, 0.0f, 1.0f}, spec_cone = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -1360,6 +1366,8 @@ constexpr uint64_t kGroup16Pixels = 1u << 14, kGroup4Pixels = 1u << 19;
 // rounds of four waves per SIMD (whole RGBA16F ambient-occlusion frame with
 // one / four waves: 320x180 450 / 399 us, 640x360 498 / 482, 960x540 615 / 615,
 // 1280x720 771 / 802, 1920x1080 1212 / 1334: the set-up is repeated per wave).
+// Modes without diffuse cones have nothing to spread and keep one wave per tile
+// (the albedo of 960x540: 10 us, 19 with four waves).
 constexpr unsigned kWideTiles = 256, kSplitTiles = 8192;
 
 // Workgroups of one k_trace launch: 2^20 (an 8192x8192 image), well below the
@@ -1383,7 +1391,8 @@ static void launch_diffuse(hipStream_t s, const typename Vol<kHalf>::T* vol, con
                            const vct_gbuffer* g, float4* out_d, float4* out_s, unsigned long long* samples)
 {
     const unsigned tiles = 4u * ((g->width + 15) / 16) * ((g->height + 15) / 16);
-    if (tiles <= kWideTiles) launch_diffuse<kHalf, kSpecPass, 16>(s, vol, P, g, out_d, out_s, samples);
+    if (!wants_diffuse(P)) launch_diffuse<kHalf, kSpecPass, 1>(s, vol, P, g, out_d, out_s, samples);
+    else if (tiles <= kWideTiles) launch_diffuse<kHalf, kSpecPass, 16>(s, vol, P, g, out_d, out_s, samples);
     else if (tiles <= kSplitTiles) launch_diffuse<kHalf, kSpecPass, 4>(s, vol, P, g, out_d, out_s, samples);
     else launch_diffuse<kHalf, kSpecPass, 1>(s, vol, P, g, out_d, out_s, samples);
 }
@@ -1562,7 +1571,9 @@ extern "C" vct_status vct_svo_trace(vct_ctx* c, vct_stream stream, const vct_gbu
                            (float4*)diffuse_out, (float4*)specular_out, samples_out);
     };
     const size_t lds = (P.cones32 ? 33u : 17u) * 64u * sizeof(f4);
-    if (4u * tiles <= kWideTiles) launch(k_svo_trace<16>, 4u * tiles, 1024, lds);
+    // the specular cone alone is one wave's work: no split without diffuse cones
+    if (!wants_diffuse(P)) launch(k_svo_trace<1>, tiles, 256, 0);
+    else if (4u * tiles <= kWideTiles) launch(k_svo_trace<16>, 4u * tiles, 1024, lds);
     else if (4u * tiles <= kSplitTiles) launch(k_svo_trace<4>, 4u * tiles, 256, lds);
     else launch(k_svo_trace<1>, tiles, 256, 0);
     VCT_HIP(hipGetLastError());
