@@ -1105,7 +1105,9 @@ __global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void k_svo_trace(
     if (surface) {
         pixel_in(P, idx, px, py, depth, g_diffuse, g_normal, g_specular, g_emission, I);
         want_spec = wants_specular(P, I);
-        for (int j = kWaves == 1 ? 0 : wave; j <= ncones; j += kWaves) {
+        // cones [first, last], 0 the specular one
+        const int first = want_spec ? 0 : 1, last = want_diffuse ? ncones : 0;
+        for (int j = kWaves == 1 ? first : wave; j <= last; j += kWaves) {
             float dir[3], ct = 0.0f, aperture = P.cones32 ? 0.628319f : 0.872665f, factor = P.step_factor;
             if (j == 0) {
                 if (!want_spec) continue;
@@ -1119,7 +1121,7 @@ __global__ __launch_bounds__(kWaves == 1 ? 256 : 64 * kWaves) void k_svo_trace(
             } else {
                 const float* d = P.cones32 ? c_dirs32[j - 1] : c_dirs16[j - 1];
                 ct = cone_cos(d);
-                if (!want_diffuse || ct < 0.0f) continue;
+                if (ct < 0.0f) continue;
                 for (int k = 0; k < 3; ++k) dir[k] = d[k];
             }
             const f4 c = svo_trace_cone(pool, P, S, I.start, dir, aperture, 30.0f, I.min_level, factor, steps);
