@@ -21,6 +21,8 @@ static std::map<const void*, std::string> names;
 static std::string launched;  // the names of the kernels launched, a blank after each
 static std::string failing;   // a launch of a kernel with this in its name fails
 static int last_error = 0, capturing = 0;
+static int waits = 0;                    // waits of the host for the stream
+static unsigned long long counted = 0;   // what every 8-byte read from the device finds
 static dim3 grid_, block_;
 static size_t shared_;
 static void* stream_;
@@ -75,14 +77,29 @@ int hipMemset(void* p, int v, size_t n)
     memset(p, v, n);
     return 0;
 }
-int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*)
+int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void*)
 {
-    memcpy(d, s, n);
+    memcpy(d, kind == 2 && n == 8 ? &counted : s, n);
     return 0;
 }
 int hipGetDevice(int* d) { return *d = 0; }
+int hipGetStreamDeviceId(void*) { return 0; }
+int hipDeviceGetAttribute(int* v, int, int)
+{
+    *v = 64;
+    return 0;
+}
+int hipGetDevicePropertiesR0600(void* p, int)
+{
+    memset(p, 0, 1472);  // the size of the properties
+    return 0;
+}
 int hipDeviceSynchronize() { return 0; }
-int hipStreamSynchronize(void*) { return 0; }
+int hipStreamSynchronize(void*)
+{
+    ++waits;
+    return 0;
+}
 int hipGetSymbolAddress(void** p, const void*)
 {
     static char c;

@@ -722,14 +722,17 @@ vct_status vct_svo_build(vct_ctx* c, vct_stream stream)
     uint2* pool = (uint2*)c->svo.pool.ptr;
     const uint2* frags = (const uint2*)c->svo.frags.ptr;
     // sizes per depth, then the pool
-    unsigned long long reached[kSvoMaxDepth] = {};  // nodes that some fragment reaches
+    unsigned long long reached[kSvoMaxDepth] = {};  // nodes that some fragment reaches, but the leaves
     if (nfrag) {
         if (L <= 10) VCT_TRY(svo_sort<uint32_t>(c, s, frags, nfrag, L, half));
         else VCT_TRY(svo_sort<unsigned long long>(c, s, frags, nfrag, L, half));
-        if (!c->pinned_word) VCT_HIP(hipHostMalloc(&c->pinned_word, kPinnedWordBytes, hipHostMallocDefault));
-        VCT_HIP(hipMemcpyAsync(c->pinned_word, c->totals.ptr, 8u * L, hipMemcpyDeviceToHost, s));
-        VCT_HIP(hipStreamSynchronize(s));
-        for (uint32_t e = 0; e < L; ++e) reached[e] = ((volatile unsigned long long*)c->pinned_word)[e];
+        // the leaves' number is not needed: an octree of one level waits for nothing
+        if (L > 1) {
+            if (!c->pinned_word) VCT_HIP(hipHostMalloc(&c->pinned_word, kPinnedWordBytes, hipHostMallocDefault));
+            VCT_HIP(hipMemcpyAsync(c->pinned_word, c->totals.ptr, 8u * (L - 1), hipMemcpyDeviceToHost, s));
+            VCT_HIP(hipStreamSynchronize(s));
+        }
+        for (uint32_t e = 0; e + 1 < L; ++e) reached[e] = ((volatile unsigned long long*)c->pinned_word)[e];
     }
     // depth e's nodes: the eight of the root, then eight per node reached above
     std::vector<uint32_t> level_begin, level_num;
